@@ -153,7 +153,11 @@ hipError_t LaunchSetModes(const Ctx &c, const int64_t *keys, const double2 *coef
                           int64_t m, hipStream_t s);
 hipError_t LaunchGetCoefs(const Ctx &c, double2 *out, int64_t m, hipStream_t s);
 // BinInFreq on a caller's rows x B matrix; limbs: rows x B x 4 integers and
-// emax one int of scratch (the exact per-bin term sums).
+// emax two ints of scratch (the exact per-bin term sums).  emax[0] starts as
+// kNoTerms (four equal bytes, so that a byte fill sets it) and every call
+// leaves it so.
+constexpr int kNoTermsByte = 0x80;
+constexpr int32_t kNoTerms = int32_t(0x80808080u);
 hipError_t LaunchBinInFreqDirect(int64_t n, int64_t mask, const BParams &bp,
                                  const DevTf &tf, int64_t q, const int64_t *k0,
                                  const double2 *coef, int64_t m, double2 *out,

@@ -14,6 +14,8 @@
 // identify/estimate by transcendental latency.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace mpsft {
@@ -1986,46 +1988,58 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
 }
 
 // BinInFreqV1 (src/binner.cc:565-591) on a caller-owned bin matrix (rows x
-// B, row stride B), one thread per mode, with each bin's terms summed
-// exactly as in the solve (TermGrid) so the result does not depend on the
-// order of the modes or of the threads: a pass for the grid exponent (the
-// largest term component over all modes, by atomicMax), a pass adding the
-// limbs into limbs[(row B + bin) kLimbs ...], and one subtracting each
+// B, row stride B), with each bin's terms summed exactly as in the solve
+// (TermGrid) so the result does not depend on the order of the modes or of
+// the threads: a pass for the grid exponent (by atomicMax), a pass adding
+// the limbs into limbs[(row B + bin) kLimbs ...], and one subtracting each
 // bin's sum.
-template <typename Fn>
-__device__ __forceinline__ void DirectTerms(int64_t n, int64_t mask, const BParams &bp,
-                                            const DevTf &tf, int64_t q, int64_t k0s,
-                                            double2 coef, Fn fn) {
+//
+// Bound by latency: a term costs two erf and two sincospi, 2 x 4 integer
+// atomics follow, and there are few modes.  So a thread takes one (mode,
+// bit), rows 2 bit + 1 and 2 bit + 2 (and row 0 for bit 0), and recomputes
+// the mode's base factor, rather than walking all rows of a mode: 500 modes
+// at n = 2^22, B = 1001 (27 rows) are 26 workgroups instead of 2, and the
+// call's passes went 58.1 -> 15.6 us.  The grid exponent comes from max |coef| wf alone (a unit
+// phase times it bounds every component within a factor sqrt(2)), so its
+// pass needs no phases and shares a launch with the clear of the limbs.
+struct DirectMode {
+  int64_t k0, k1;
+  int32_t bin;
+  double2 cw;  // coef wf
+};
+__device__ __forceinline__ DirectMode DirectBase(int64_t n, int64_t mask, const BParams &bp,
+                                                 const DevTf &tf, int64_t k0s, double2 coef) {
+  DirectMode d;
   const int32_t B = bp.B;
-  const int64_t k0 = ModN(k0s, n, mask);
-  const int64_t k1 = ModN(tf.a * k0 + tf.b, n, mask);
-  const int32_t bin = int32_t(k1 * B / n);
-  const double xi = (double(bin) + 0.5) / double(B) - double(k1) / double(n);
-  const double wf = SampleInFreq(xi, bp.width, bp.dfreq);
-  const double2 base = Cmul(Scale(coef, wf), CisFrac(ModN(q * k1 + tf.c * k0, n, mask), n));
-  fn(0, bin, base);
-  for (int32_t bit = 0; bit < bp.bits; ++bit) {
-    const double2 g = CisFrac(ModN((int64_t(B) << bit) * k1, n, mask), n);
-    fn(2 * bit + 1, bin, Cmul(base, g));
-    fn(2 * bit + 2, bin, Cmul(base, Conj(g)));
-  }
+  d.k0 = ModN(k0s, n, mask);
+  d.k1 = ModN(tf.a * d.k0 + tf.b, n, mask);
+  d.bin = int32_t(d.k1 * B / n);
+  const double xi = (double(d.bin) + 0.5) / double(B) - double(d.k1) / double(n);
+  d.cw = Scale(coef, SampleInFreq(xi, bp.width, bp.dfreq));
+  return d;
 }
 
+// limbs[0..count) = 0 (a kernel rather than a memset), and emax[0] = the
+// exponent of the largest |coef| wf (emax[0] is kNoTerms before: from the
+// plan's creation or the previous call's last pass).
 __global__ void __launch_bounds__(kThreads)
-    k_freq_direct_max(int64_t n, int64_t mask, BParams bp, DevTf tf, int64_t q,
-                      const int64_t *k0s, const double2 *coefs, int64_t m, int32_t *emax) {
+    k_freq_direct_max(int64_t n, int64_t mask, BParams bp, DevTf tf, const int64_t *k0s,
+                      const double2 *coefs, int64_t m, int32_t *emax, unsigned long long *limbs,
+                      int64_t count) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t gsize = int64_t(gridDim.x) * blockDim.x;
+  for (int64_t j = i; j < count; j += gsize) limbs[j] = 0ull;
   double mx = 0.0;
-  if (i < m)
-    DirectTerms(n, mask, bp, tf, q, k0s[i], coefs[i],
-                [&](int, int32_t, double2 v) { mx = fmax(mx, MaxComp(v)); });
+  for (int64_t j = i; j < m; j += gsize) {
+    const DirectMode d = DirectBase(n, mask, bp, tf, k0s[j], coefs[j]);
+    mx = fmax(mx, hypot(d.cw.x, d.cw.y));
+  }
   for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
   if ((threadIdx.x & 63) == 0 && mx > 0.0) atomicMax(emax, ilogb(mx) + 1);
 }
 
 // The grid of exponent e (every term component below 2^e); e = kNoTerms
 // when there is no nonzero term.
-constexpr int32_t kNoTerms = -(1 << 30);
 __device__ __forceinline__ TermGrid TermGridOf(int32_t e) {
   TermGrid g;
   g.any = e != kNoTerms;
@@ -2034,32 +2048,41 @@ __device__ __forceinline__ TermGrid TermGridOf(int32_t e) {
   return g;
 }
 
+// One (mode, bit) per thread.  emax[1] = emax[0] for the last pass.
 __global__ void __launch_bounds__(kThreads)
     k_freq_direct_add(int64_t n, int64_t mask, BParams bp, DevTf tf, int64_t q,
-                      const int64_t *k0s, const double2 *coefs, int64_t m, const int32_t *emax,
+                      const int64_t *k0s, const double2 *coefs, int64_t m, int32_t *emax,
                       unsigned long long *limbs) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const TermGrid g = TermGridOf(*emax);
-  if (i >= m || !g.any) return;
-  DirectTerms(n, mask, bp, tf, q, k0s[i], coefs[i], [&](int row, int32_t bin, double2 v) {
-    LimbAdd(limbs + kLimbs * (int64_t(row) * bp.B + bin), v, g);
-  });
+  const int32_t e = emax[0];
+  if (i == 0) emax[1] = e;
+  const TermGrid g = TermGridOf(e);
+  const int64_t work = m * bp.bits;
+  if (!g.any) return;
+  for (int64_t j = i; j < work; j += int64_t(gridDim.x) * blockDim.x) {
+    // modes over the lanes (coalesced reads), bits over the blocks
+    const int32_t bit = int32_t(j / m);
+    const int64_t mi = j - int64_t(bit) * m;
+    const DirectMode d = DirectBase(n, mask, bp, tf, k0s[mi], coefs[mi]);
+    const double2 base = Cmul(d.cw, CisFrac(ModN(q * d.k1 + tf.c * d.k0, n, mask), n));
+    const double2 t = CisFrac(ModN((int64_t(bp.B) << bit) * d.k1, n, mask), n);
+    unsigned long long *acc = limbs + kLimbs * (int64_t(2 * bit + 1) * bp.B + d.bin);
+    if (bit == 0) LimbAdd(limbs + kLimbs * int64_t(d.bin), base, g);
+    LimbAdd(acc, Cmul(base, t), g);
+    LimbAdd(acc + kLimbs * int64_t(bp.B), Cmul(base, Conj(t)), g);
+  }
 }
 
+// out -= the bins' sums; emax[0] is left ready for the next call.
 __global__ void __launch_bounds__(kThreads)
-    k_freq_direct_sub(const unsigned long long *limbs, const int32_t *emax, int64_t count,
+    k_freq_direct_sub(const unsigned long long *limbs, int32_t *emax, int64_t count,
                       double2 *out) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const TermGrid g = TermGridOf(*emax);
-  if (i < count && g.any) out[i] = Sub(out[i], LimbValue(limbs + kLimbs * i, g));
-}
-
-// limbs[0..count) = 0 and *emax = kNoTerms (a kernel rather than a memset).
-__global__ void __launch_bounds__(kThreads)
-    k_freq_direct_clear(unsigned long long *limbs, int64_t count, int32_t *emax) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  for (int64_t j = i; j < count; j += int64_t(gridDim.x) * blockDim.x) limbs[j] = 0ull;
-  if (i == 0) *emax = kNoTerms;
+  const TermGrid g = TermGridOf(emax[1]);
+  if (i == 0) emax[0] = kNoTerms;
+  if (!g.any) return;
+  for (int64_t j = i; j < count; j += int64_t(gridDim.x) * blockDim.x)
+    out[j] = Sub(out[j], LimbValue(limbs + kLimbs * j, g));
 }
 
 __global__ void __launch_bounds__(kThreads)
@@ -3050,12 +3073,10 @@ hipError_t LaunchBinInFreqDirect(int64_t n, int64_t mask, const BParams &bp,
                                  unsigned long long *limbs, int32_t *emax, hipStream_t s) {
   if (m <= 0) return hipSuccess;
   const int64_t bins = int64_t(1 + 2 * bp.bits) * bp.B;
-  hipLaunchKernelGGL(k_freq_direct_clear, dim3(Blocks(kLimbs * bins)), dim3(kThreads), 0, s, limbs,
-                     kLimbs * bins, emax);
-  hipLaunchKernelGGL(k_freq_direct_max, dim3(Blocks(m)), dim3(kThreads), 0, s, n, mask, bp, tf, q,
-                     k0, coef, m, emax);
-  hipLaunchKernelGGL(k_freq_direct_add, dim3(Blocks(m)), dim3(kThreads), 0, s, n, mask, bp, tf, q,
-                     k0, coef, m, emax, limbs);
+  hipLaunchKernelGGL(k_freq_direct_max, dim3(Blocks(std::max(kLimbs * bins, m))), dim3(kThreads), 0,
+                     s, n, mask, bp, tf, k0, coef, m, emax, limbs, kLimbs * bins);
+  hipLaunchKernelGGL(k_freq_direct_add, dim3(Blocks(m * bp.bits)), dim3(kThreads), 0, s, n, mask, bp,
+                     tf, q, k0, coef, m, emax, limbs);
   hipLaunchKernelGGL(k_freq_direct_sub, dim3(Blocks(bins)), dim3(kThreads), 0, s, limbs, emax, bins,
                      out);
   return hipGetLastError();

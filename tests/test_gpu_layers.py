@@ -1,0 +1,34 @@
+"""The layers' kernels at the edges of their tiles and launches, against the
+CPU oracle (1e-12 of the largest value, as in the parity tests)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+def _tf(gpu, orc, n, seed):
+    orc.seed(seed)
+    tf = orc.transform_draw(n)
+    return tf, gpu.transform_make(n, int(tf[0]), int(tf[1]), int(tf[2]))
+
+
+@pytest.mark.parametrize("n,bins,m", [(4099, 3, 1), (1 << 12, 4095, 64), (1 << 16, 101, 256),
+                                      (1 << 18, 2001, 257), (1000003, 501, 1025)])
+def test_bin_in_freq_edges(gpu, orc, n, bins, m):
+    """One thread per (mode, bit): mode counts at and beyond a workgroup,
+    bits from 1 (n / B < 2) up; calls in a row on one plan, one of them with
+    zero coefficients (no grid) and one of tiny ones, share its scratch."""
+    rng = np.random.default_rng(n + m)
+    bits = orc.num_bits(n, bins)
+    tf_o, tf = _tf(gpu, orc, n, m)
+    keys = rng.choice(n, m, replace=False).astype(np.int64)
+    plan = gpu.Plan(n, bins, 1e-6, bits)
+    for scale in (1.0, 0.0, 1e-30, 1.0):
+        coefs = scale * (rng.standard_normal(m) + 1j * rng.standard_normal(m))
+        base = scale * (rng.standard_normal((1 + 2 * bits, bins)) + 1j)
+        ref, got = base.copy(), base.copy()
+        orc.bin_in_freq(keys.astype(np.int32), coefs, n, bins, 1e-6, bits, tf_o, 77, ref, version=1)
+        plan.bin_in_freq(keys, coefs, tf, 77, got)
+        assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
