@@ -1203,6 +1203,18 @@ int Engine::Adjoint(const int64_t *keys, const void *grad, int64_t m, void *out,
   return MPSFT_OK;
 }
 
+OneShot Engine::MakeOneShot(int32_t mode, const void *x, const BParams &bp, const DevTf &tf,
+                            const int64_t *qs, int32_t trials) const {
+  OneShot o{};
+  o.x = x;
+  o.tf = tf;
+  for (int32_t t = 0; t < trials; ++t) o.q[t] = PosMod(qs[t], n_);
+  o.bp = bp;
+  o.mode = mode;
+  o.trials = trials;
+  return o;
+}
+
 int Engine::IterateOnce(const void *x, const mpsft_iterate_options &opt, const DevTf &tf,
                         const int64_t *qs, int32_t *found, hipStream_t s) {
   Drain();
@@ -1222,29 +1234,16 @@ int Engine::IterateOnce(const void *x, const mpsft_iterate_options &opt, const D
   if (rc != MPSFT_OK) return rc;
   rc = Reserve(opt.trials, bs);
   if (rc != MPSFT_OK) return rc;
-  bool grown = false;
-  rc = GrowTransforms(1, &grown);
-  if (rc != MPSFT_OK) return rc;
   tf_valid_ = false;
-  std::vector<int64_t> hq(trials_cap_, 0);
-  for (int32_t t = 0; t < opt.trials; ++t) hq[t] = PosMod(qs[t], n_);
-  HIP_OK(hipMemcpyAsync(d_tfs_, &tf, sizeof(DevTf), hipMemcpyHostToDevice, s));
-  HIP_OK(hipMemcpyAsync(d_qs_, hq.data(), hq.size() * sizeof(int64_t), hipMemcpyHostToDevice, s));
-  Ctx c = MakeCtx();
-  InitArgs a{};
-  a.x = x;
-  a.mode = kModeIterate;
-  a.B = opt.bins;
-  a.trials = opt.trials;
-  a.max_stale = 1;
-  a.max_iter = 1;
-  a.keep_modes = 1;
-  a.bin_thr = opt.bin_threshold;
-  a.sv_thr = opt.sv_threshold;
-  a.win_thr = opt.window_threshold;
-  HIP_OK(LaunchInit(c, a, s));
-  rc = LaunchIteration(c, 0, s);
+  const Ctx c = MakeCtx();
+  OneShot o = MakeOneShot(kModeIterate, x, hbtab_[opt.bins], tf, qs, opt.trials);
+  o.bin_thr = opt.bin_threshold;
+  o.sv_thr = opt.sv_threshold;
+  o.win_thr = opt.window_threshold;
+  HIP_OK(LaunchBinTimeOnce(c, o, TilesCap(), LdsBinTime(c.mixed != 0), s));
+  rc = LaunchFft(c, 0, s);
   if (rc != MPSFT_OK) return rc;
+  HIP_OK(LaunchIdentify(c, 0, IdentifyBlocks(), s));
   rc = ReadState(s);
   if (rc != MPSFT_OK) return rc;
   *found = h_state_->found_iter[0];
@@ -1266,27 +1265,14 @@ int Engine::BinOnly(const void *x, int32_t B, double delta, int32_t bits, const 
   // out's layout is rows x B: the engine's row stride must be B (a larger
   // trials_cap_ from an earlier IdentifyOnly leaves trial 0's rows alone)
   if (B_cap_ != B || rows_cap_ != 1 + 2 * bits) return MPSFT_ERR_SHAPE;
-  bool grown = false;
-  rc = GrowTransforms(1, &grown);
-  if (rc != MPSFT_OK) return rc;
   tf_valid_ = false;
-  const int64_t hq = PosMod(q, n_);
-  HIP_OK(hipMemcpyAsync(d_tfs_, &tf, sizeof(DevTf), hipMemcpyHostToDevice, s));
-  HIP_OK(hipMemcpyAsync(d_qs_, &hq, sizeof(int64_t), hipMemcpyHostToDevice, s));
   A_override_ = out;
   Ctx c = MakeCtx();
   if (d_wtab_ && wtab_B_ == B) c.wtab = d_wtab_;
-  InitArgs a{};
-  a.x = x;
-  a.mode = kModeBinOnly;
-  a.B = B;
-  a.trials = 1;
-  a.max_stale = 1;
-  a.max_iter = 1;
-  a.bits_override = bits;
-  a.win_thr = 1;
-  HIP_OK(LaunchInit(c, a, s));
-  HIP_OK(LaunchBinTime(c, 0, TilesCap(), LdsBinTime(c.mixed != 0), s));
+  OneShot o = MakeOneShot(kModeBinOnly, x, hbtab_[B], tf, &q, 1);
+  o.bp.bits = bits;
+  o.win_thr = 1;
+  HIP_OK(LaunchBinTimeOnce(c, o, TilesCap(), LdsBinTime(c.mixed != 0), s));
   rc = LaunchFft(c, 0, s);
   A_override_ = nullptr;
   if (rc != MPSFT_OK) return rc;
@@ -1320,36 +1306,21 @@ int Engine::IdentifyOnly(const double2 *A, int32_t trials, int32_t B, double del
   // A's layout is [trial][row][bin] with rows x B per trial: the engine's
   // strides must be exactly those.
   if (B_cap_ != B || rows_cap_ != 1 + 2 * bits) return MPSFT_ERR_SHAPE;
-  bool grown = false;
-  rc = GrowTransforms(1, &grown);
-  if (rc != MPSFT_OK) return rc;
   tf_valid_ = false;
-  std::vector<int64_t> hq(trials_cap_, 0);
-  for (int32_t t = 0; t < trials; ++t) hq[t] = PosMod(qs[t], n_);
   if (!d_idout_ && Alloc(&d_idout_, 1) != MPSFT_OK) return MPSFT_ERR_NOMEM;
-  HIP_OK(hipMemcpyAsync(d_tfs_, &tf, sizeof(DevTf), hipMemcpyHostToDevice, s));
-  HIP_OK(hipMemcpyAsync(d_qs_, hq.data(), hq.size() * sizeof(int64_t), hipMemcpyHostToDevice, s));
-  HIP_OK(hipMemcpyAsync(d_idout_, &out, sizeof(IdOut), hipMemcpyHostToDevice, s));
   A_override_ = const_cast<double2 *>(A);
   Ctx c = MakeCtx();
   A_override_ = nullptr;
   c.idout = d_idout_;
-  InitArgs a{};
-  a.x = A;  // not read: no gather runs
-  a.mode = kModeIterate;
-  a.B = B;
-  a.trials = trials;
-  a.max_stale = 1;
-  a.max_iter = 1;
-  a.bits_override = bits;
-  a.bin_thr = bin_thr;
-  a.sv_thr = sv_thr;
-  a.win_thr = win_thr;
-  HIP_OK(LaunchReset(c, a, s));
-  HIP_OK(LaunchPublish(c, 0, s));
+  // A stands for x, which is not read: no gather runs
+  OneShot o = MakeOneShot(kModeIterate, A, hbtab_[B], tf, qs, trials);
+  o.bp.bits = bits;
+  o.bin_thr = bin_thr;
+  o.sv_thr = sv_thr;
+  o.win_thr = win_thr;
+  HIP_OK(LaunchPublishOnce(c, o, out, d_idout_, s));
   HIP_OK(LaunchIdentify(c, 0, IdentifyBlocks(), s));
-  // the host copies of out and the q's are read by the copies above
-  HIP_OK(hipStreamSynchronize(s));
+  HIP_OK(hipStreamSynchronize(s));  // the outputs are ready on return
   return MPSFT_OK;
 }
 

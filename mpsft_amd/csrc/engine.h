@@ -34,6 +34,7 @@
 namespace mpsft {
 
 struct InitArgs;
+struct OneShot;
 
 constexpr int kThreads = 256;      // workgroup size of most kernels
 constexpr int kFftThreads = 256;   // workgroup size of k_bin_fft
@@ -275,6 +276,10 @@ class Engine {
   TfUpload *defer_upload_ = nullptr;
   int GrowTransforms(int32_t count, bool *grown);
   Ctx MakeCtx() const;
+  // One iteration's parameters (q's reduced modulo n); thresholds are the
+  // caller's to set.
+  OneShot MakeOneShot(int32_t mode, const void *x, const BParams &bp, const DevTf &tf,
+                      const int64_t *qs, int32_t trials) const;
   int LaunchIteration(const Ctx &c, int parity, hipStream_t s, bool big = true);
   int LaunchFft(const Ctx &c, int parity, hipStream_t s, bool big = true);
   int EnsureGraph(int32_t iters, hipStream_t s);

@@ -17,6 +17,25 @@ struct InitArgs {
   double bin_thr, sv_thr, win_thr;
 };
 
+// One iteration with explicit parameters (a plan call or Iterate), passed to
+// its first kernel by value: nothing is uploaded.  bp carries the call's own
+// bits.
+struct OneShot {
+  const void *x;
+  DevTf tf;
+  int64_t q[kMaxTrials];
+  BParams bp;
+  int32_t mode, trials;
+  double bin_thr, sv_thr, win_thr;
+};
+// k_bin_time for a OneShot, which also publishes it (parity 0) for the bin
+// FFT and k_identify.
+hipError_t LaunchBinTimeOnce(const Ctx &c, const OneShot &o, int32_t tiles, size_t lds,
+                             hipStream_t s);
+// A OneShot published without a gather-fold, and *idout = out.
+hipError_t LaunchPublishOnce(const Ctx &c, const OneShot &o, const IdOut &out, IdOut *idout,
+                             hipStream_t s);
+
 hipError_t LaunchBuildTwiddles(double2 *tw, hipStream_t s);
 hipError_t LaunchBuildTables(const int32_t *blist, int32_t nb, const BParams *btab,
                              double2 *table, const double2 *tw, int32_t M_cap,
@@ -39,9 +58,6 @@ hipError_t LaunchBinFft(const Ctx &c, int parity, size_t lds, hipStream_t s);
 // The four-step bin FFT (B > kMaxLdsBins): three kernels.
 hipError_t LaunchBigFft(const Ctx &c, int parity, hipStream_t s);
 hipError_t LaunchIdentify(const Ctx &c, int parity, int32_t blocks, hipStream_t s);
-// Publishes the next iteration's parameters in slot `parity` (k_bin_time's
-// first workgroup alone: no gather, no terms of found modes).
-hipError_t LaunchPublish(const Ctx &c, int parity, hipStream_t s);
 
 // The batched form: per-stage launches over every signal of a batch.
 // BatchWork (device) is rewritten by each batched iteration's plan: per

@@ -562,9 +562,11 @@ struct Lags {
 // Workgroups below kPrepBlocks instead compute the BinInFreq terms of every
 // found mode for this iteration.
 // blk: this workgroup's block index within the signal's launch.
+// x, qs: the signal and the iteration's q per trial.
 template <typename Tx, bool kNt = true>
-__device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, int32_t trials,
-                                         int32_t tile, double2 *lds);
+__device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, const void *xv,
+                                         const int64_t *qs, int32_t trials, int32_t tile,
+                                         double2 *lds);
 
 // The BinInFreq factor of mode k0 (k1 = its image under the transform) in
 // row 0 for offset q: wf(xi) e^{2 pi i (q k1 + c k0)/n}, and its bin.  Every
@@ -592,8 +594,8 @@ __device__ __forceinline__ double2 BitTwiddle(const Ctx &c, int32_t B, int bit, 
 // g = e^{2 pi i (B 2^bit k1)/n}; the terms are coef base (row 0),
 // coef (base g) (row 2bit+1) and coef (base conj(g)) (row 2bit+2).
 // Workgroup blk of nblk.
-__device__ __forceinline__ void FreqTerms(const Ctx &c, const IterParams &ip, int32_t trials,
-                                          int32_t blk, int32_t nblk) {
+__device__ __forceinline__ void FreqTerms(const Ctx &c, const IterParams &ip, const int64_t *qs,
+                                          int32_t trials, int32_t blk, int32_t nblk) {
   const int32_t B = ip.B, bits = ip.bits;
   const DevTf tf = ip.tf;
   const int64_t n = c.n, mask = c.mask;
@@ -604,7 +606,7 @@ __device__ __forceinline__ void FreqTerms(const Ctx &c, const IterParams &ip, in
     const int32_t mi = int32_t(i - int64_t(trial) * cnt);
     const int64_t k0 = c.keys[mi];
     const double2 cf = c.coef[k0];
-    const int64_t q = c.qs[int64_t(ip.it) * c.trials_cap + trial];
+    const int64_t q = qs[trial];
     const int64_t k1 = ModN(tf.a * k0 + tf.b, n, mask);
     int32_t bin;
     const double2 base = FreqBase(c, ip, q, k0, k1, &bin);
@@ -619,6 +621,11 @@ __device__ __forceinline__ void FreqTerms(const Ctx &c, const IterParams &ip, in
   }
 }
 
+// The q per trial of a solve's iteration it.
+__device__ __forceinline__ const int64_t *IterQs(const Ctx &c, int32_t it) {
+  return c.qs + int64_t(it) * c.trials_cap;
+}
+
 template <typename Tx>
 __device__ __forceinline__ void BinTimeBody(const Ctx &c, int p, int blk, double2 *lds) {
   const DevState *st = c.st;
@@ -628,20 +635,19 @@ __device__ __forceinline__ void BinTimeBody(const Ctx &c, int p, int blk, double
   if (blk == 0 && threadIdx.x == 0) PublishIteration(c, p, ip, lc);
   if (ip.done) return;
   const int32_t trials = st->trials;
-  if (blk < kPrepBlocks) {
-    FreqTerms(c, ip, trials, blk, kPrepBlocks);
-    return;
-  }
-
-  TileFold<Tx>(c, ip, trials, blk - kPrepBlocks, lds);
+  const int64_t *qs = IterQs(c, ip.it);
+  if (blk < kPrepBlocks)
+    FreqTerms(c, ip, qs, trials, blk, kPrepBlocks);
+  else
+    TileFold<Tx>(c, ip, st->x, qs, trials, blk - kPrepBlocks, lds);
 }
 
 // The gather-fold of one tile (trial, block of R residues) of an iteration
 // with parameters ip (see BinTimeBody).
 template <typename Tx, bool kNt>
-__device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, int32_t trials,
-                                         int32_t tile, double2 *lds) {
-  const DevState *st = c.st;
+__device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, const void *xv,
+                                         const int64_t *qs, int32_t trials, int32_t tile,
+                                         double2 *lds) {
   const int32_t B = ip.B, f = ip.f, bits = ip.bits, p2 = ip.p2, rows = ip.rows;
   const DevTf tf = ip.tf;
   const int64_t n = c.n, mask = c.mask;
@@ -655,8 +661,8 @@ __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, int
   const int32_t rho0 = (tile - trial * nblk) * R;
   const int32_t nrho = min(R, B - rho0);
   const Lags L(bits, f);
-  const int64_t q = c.qs[int64_t(ip.it) * c.trials_cap + trial];
-  const Tx *x = static_cast<const Tx *>(st->x);
+  const int64_t q = qs[trial];
+  const Tx *x = static_cast<const Tx *>(xv);
 
   // [nlam][R] samples as stored in x (complex64 samples take half the LDS
   // and widen exactly at use), then [f][R] taps and [kThreads] partial sums
@@ -753,6 +759,59 @@ template <typename Tx>
 __global__ void __launch_bounds__(kThreads) k_bin_time(Ctx c, int p) {
   HIP_DYNAMIC_SHARED(double2, lds)
   BinTimeBody<Tx>(c, p, blockIdx.x, lds);
+}
+
+// One iteration with explicit parameters (a plan's BinInTime, Iterate).
+// The parameters come with the launch: two small uploads and a k_init launch
+// before the gather-fold took longer than the fold of a small bin matrix
+// (n = 2^16, B = 101: 20.5 us per call with them, 12.7 without; identify
+// and estimate at n = 2^20, B = 801, three uploads less: 39.5 -> 26.7 us).
+__device__ __forceinline__ void OnceParams(const Ctx &c, const OneShot &o, IterParams *ip) {
+  FillParams(ip, o.bp, o.bp.bits);
+  ip->bin_thr = o.bin_thr;
+  ip->sv_thr = o.sv_thr;
+  ip->tf = o.tf;
+  ip->it = 0;
+  // Iterate on a map that overflowed earlier does nothing (and reports it)
+  ip->done = o.mode == kModeIterate && (c.st->flags & kFlagOverflow) ? 1 : 0;
+}
+
+// The loop state as k_bin_fft, k_identify and the host read it (slot 0).
+__device__ __forceinline__ void OncePublish(const Ctx &c, const OneShot &o, const IterParams &ip) {
+  DevState *st = c.st;
+  st->x = o.x;
+  st->mode = o.mode;
+  st->trials = o.trials;
+  st->win_thr = o.win_thr;
+  st->found_iter[0] = 0;
+  st->iters = 0;
+  st->stop_stale = 0;
+  st->L[0] = LoopCounters{0, 0, ip.done, 0};
+  st->L[1] = LoopCounters{-1, 0, 0, 0};
+  st->P[0] = ip;
+  for (int t = 0; t < o.trials; ++t) st->P[0].q[t] = o.q[t];
+}
+
+template <typename Tx>
+__global__ void __launch_bounds__(kThreads) k_bin_time_once(Ctx c, OneShot o) {
+  HIP_DYNAMIC_SHARED(double2, lds)
+  const int32_t blk = blockIdx.x;
+  IterParams ip;
+  OnceParams(c, o, &ip);
+  if (blk == 0 && threadIdx.x == 0) OncePublish(c, o, ip);
+  if (ip.done) return;
+  if (blk < kPrepBlocks)
+    FreqTerms(c, ip, o.q, o.trials, blk, kPrepBlocks);
+  else
+    TileFold<Tx>(c, ip, o.x, o.q, o.trials, blk - kPrepBlocks, lds);
+}
+
+__global__ void k_publish_once(Ctx c, OneShot o, IdOut out, IdOut *idout) {
+  IterParams ip;
+  OnceParams(c, o, &ip);
+  ip.done = 0;
+  OncePublish(c, o, ip);
+  *idout = out;
 }
 
 // ---------------------------------------------------------------------------
@@ -1840,7 +1899,7 @@ __global__ void __launch_bounds__(kThreads)
     }
     return;
   }
-  TileFold<Tx>(c, ip, trials, pb - kPrepBlocks, lds);
+  TileFold<Tx>(c, ip, st->x, IterQs(c, ip.it), trials, pb - kPrepBlocks, lds);
 }
 
 template <int kPaths>
@@ -2285,11 +2344,12 @@ __device__ __forceinline__ void BinTimeUnit(const Ctx &c, int p, int32_t unit, d
   const DevState *st = c.st;
   const IterParams &ip = st->P[p];
   const int32_t trials = st->trials;
+  const int64_t *qs = IterQs(c, ip.it);
   const int32_t nprep = PrepUnits(int64_t(min(st->count, c.cap)) * trials);
   if (unit < nprep)
-    FreqTerms(c, ip, trials, unit, nprep);
+    FreqTerms(c, ip, qs, trials, unit, nprep);
   else
-    TileFold<Tx, false>(c, ip, trials, unit - nprep, lds);
+    TileFold<Tx, false>(c, ip, st->x, qs, trials, unit - nprep, lds);
 }
 
 template <typename Tx>
@@ -3032,8 +3092,19 @@ hipError_t LaunchLateIteration(const Ctx &c, int parity, int32_t nb_ident, int32
   return hipGetLastError();
 }
 
-hipError_t LaunchPublish(const Ctx &c, int parity, hipStream_t s) {
-  hipLaunchKernelGGL(k_bin_time<double2>, dim3(1), dim3(kThreads), 0, s, c, parity);
+hipError_t LaunchBinTimeOnce(const Ctx &c, const OneShot &o, int32_t tiles, size_t lds,
+                             hipStream_t s) {
+  const dim3 grid(kPrepBlocks + tiles);
+  if (c.mixed)
+    hipLaunchKernelGGL(k_bin_time_once<float2>, grid, dim3(kThreads), lds, s, c, o);
+  else
+    hipLaunchKernelGGL(k_bin_time_once<double2>, grid, dim3(kThreads), lds, s, c, o);
+  return hipGetLastError();
+}
+
+hipError_t LaunchPublishOnce(const Ctx &c, const OneShot &o, const IdOut &out, IdOut *idout,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(k_publish_once, dim3(1), dim3(1), 0, s, c, o, out, idout);
   return hipGetLastError();
 }
 

@@ -32,3 +32,23 @@ def test_bin_in_freq_edges(gpu, orc, n, bins, m):
         orc.bin_in_freq(keys.astype(np.int32), coefs, n, bins, 1e-6, bits, tf_o, 77, ref, version=1)
         plan.bin_in_freq(keys, coefs, tf, 77, got)
         assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
+
+
+def test_iterate_after_overflow_changes_nothing(gpu):
+    """A map that overflowed its capacity stays as it is: the one-launch
+    parameters of Iterate carry the stop to the later kernels."""
+    from mpsft_amd.signals import make_signal
+    n, k = 1 << 14, 40
+    x, _ = make_signal(n, k, 1e-6, seed=3)
+    s = gpu.Solver(n, gpu.solve_options(k, 1e-6), capacity=4)
+    opt = gpu.iterate_options(101, trials=1, bin_threshold=3e-7, window_threshold=0.1,
+                              sv_threshold=1e-7)
+    xd = s.upload(x)
+    for rep in range(2):
+        tf = gpu.transform_make(n, 2 * rep + 5, 1, 2)
+        with pytest.raises(gpu.MpsftError) as e:
+            s.iterate(xd, opt, tf, [7])
+        assert e.value.status == 6
+        got = s.modes_dict()
+        assert len(got) == 4 and (rep == 0 or got == first)
+        first = got
