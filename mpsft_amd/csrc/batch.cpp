@@ -72,6 +72,7 @@ Batch::Batch(int32_t count, const int64_t *n, const mpsft_solve_options *opts, i
     // 2048 tiles per trial over the batch (measured on 64 config-2 signals:
     // 512 tiles per signal 152.2, 64 per signal 144.7 us per solve)
     eng_.back()->tile_target_ = std::max(16, std::min(kTargetTiles, 2048 / count));
+    eng_.back()->batch_count_ = count;
     opts_.push_back(opts[i]);
   }
   args_.resize(count);
@@ -237,6 +238,12 @@ int Batch::Build(hipStream_t s) {
   bl_.counters = d_counters_;
   bl_.host = d_host_;
   bl_.mixed = precision_ == MPSFT_MIXED ? 1 : 0;
+  // XCD order, unless there is one signal (every XCD reads its x anyway) or
+  // its tiles are split by slices, which count on units going round robin
+  bl_.xcd_order = K > 1 ? 1 : 0;
+  for (auto &e : eng_)
+    for (const BParams &bp : e->hbtab_)
+      if (bp.slices > 1) bl_.xcd_order = 0;
 
   for (hipGraphExec_t *ge : {&graph_, &graph_small_})
     if (*ge) {

@@ -105,6 +105,16 @@ int32_t Log2(int64_t n) {
   return l;
 }
 
+// LDS of one k_bin_time tile of R residues: the samples as stored in x, the
+// taps, and the partial sums (whose place first holds the sorted order's lag
+// list and buckets, at most kSortMaxLags + kSortBuckets 16-bit words).
+size_t TileLds(const BParams &bp, int32_t nlam, size_t elem) {
+  static_assert((kSortMaxLags + kSortBuckets) * sizeof(uint16_t) <= kThreads * sizeof(double2),
+                "the lists fit the partial sums' place");
+  return (size_t(nlam) * bp.R * elem + 15) / 16 * 16 +
+         (size_t(bp.f) * bp.R + kThreads) * sizeof(double2);
+}
+
 // Transforms drawn before a solve's first launch.
 constexpr int32_t kFirstDraws = 32;
 
@@ -186,6 +196,8 @@ bool WindowParams(int64_t n, int32_t bins, double delta, BParams *bp) {
   bp->M = 1 << logM;
   bp->off = 0;
   bp->R = 1;
+  bp->G = 1;
+  bp->sorted = 0;
   bp->slices = 1;
   bp->slice_shift = 0;
   bp->width = width;
@@ -362,6 +374,36 @@ Engine::~Engine() {
   if (h_progress_) (void)hipHostFree(const_cast<int32_t *>(h_progress_));
 }
 
+// The gather-fold's tiles of one B.  G is the default width, so that a
+// residue's sum is added alike at every R.  Sorted order: batched signals
+// that do not fit the L2s (from 16 MB; 8 MB signals lose nothing to unsorted
+// tiles in XCD order, TileFold) and B of at least 256, below which a line of
+// x hardly serves two samples.  Its tiles are 8 residues wide where the
+// batch still has 384 of them (64 signals, B = 777: R = 4 467 us, R = 8 418)
+// and three fit a CU's LDS.
+void Engine::SetTile(BParams *bp, int32_t nlam) const {
+  const int32_t forced = forced_R_[bp->B >= kSmallTileB ? 0 : 1];
+  const size_t elem = precision_ == MPSFT_MIXED ? sizeof(float2) : sizeof(double2);
+  bp->slices = SlicesFor(n_, mask_, *bp);
+  bp->slice_shift = bp->slices > 1 ? Log2(n_) - 3 : 0;
+  bp->G = ResiduesPerTile(bp->B, nlam, bp->f, 0, tile_target_);
+  bp->sorted = batch_count_ > 1 && mask_ >= 0 && size_t(n_) * elem >= (size_t(16) << 20) &&
+                       bp->B >= kSmallTileB && nlam >= kThreads && nlam <= kSortMaxLags &&
+                       bp->slices == 1
+                   ? 1 : 0;
+  if (forced > 0) {
+    bp->R = ResiduesPerTile(bp->B, nlam, bp->f, forced, tile_target_);
+    return;
+  }
+  bp->R = bp->G;
+  if (!bp->sorted) return;
+  constexpr size_t kThirdLds = 160 * 1024 / 3;
+  for (bp->R = 8; bp->R > 1; bp->R /= 2)
+    if (int64_t(batch_count_) * bp->B >= 384 * int64_t(bp->R) &&
+        TileLds(*bp, nlam, elem) <= kThirdLds)
+      break;
+}
+
 // Builds the window parameters of every B in bs (for window delta) that is
 // not built yet, and for B <= kMaxLdsBins its chirp and Bluestein filter.
 int Engine::EnsureTables(const std::vector<int32_t> &bs, double delta, int32_t bits_override) {
@@ -394,9 +436,7 @@ int Engine::EnsureTables(const std::vector<int32_t> &bs, double delta, int32_t b
     if (!WindowParams(n_, B, delta, &bp)) return MPSFT_ERR_INVALID_ARG;
     if (bp.logM > kMaxLogMBig) return MPSFT_ERR_UNSUPPORTED;
     const int32_t nlam = NumLags(bits_override > 0 ? bits_override : bp.bits, bp.f);
-    bp.R = ResiduesPerTile(B, nlam, bp.f, forced_R_[B >= kSmallTileB ? 0 : 1], tile_target_);
-    bp.slices = SlicesFor(n_, mask_, bp);
-    bp.slice_shift = bp.slices > 1 ? Log2(n_) - 3 : 0;
+    SetTile(&bp, nlam);
     bp.off = 0;
     if (bp.logM <= kMaxLogM) {
       bp.off = table_used_ + need;
@@ -483,8 +523,7 @@ int Engine::SetTileResidues(int32_t R_wide, int32_t R_narrow) {
     if (!built_[B]) continue;
     BParams &bp = hbtab_[B];
     const int32_t bits = tab_bits_override_ > 0 ? tab_bits_override_ : bp.bits;
-    bp.R = ResiduesPerTile(int32_t(B), NumLags(bits, bp.f), bp.f,
-                           forced_R_[B >= size_t(kSmallTileB) ? 0 : 1], tile_target_);
+    SetTile(&bp, NumLags(bits, bp.f));
   }
   if (d_btab_)
     HIP_OK(hipMemcpy(d_btab_, hbtab_.data(), hbtab_.size() * sizeof(BParams),
@@ -505,10 +544,9 @@ int Engine::Reserve(int32_t trials, const std::vector<int32_t> &bs) {
     rc = std::max(rc, 1 + 2 * bits);
     tc = std::max(tc, (B + bp.R - 1) / bp.R * bp.slices);
     Mc = std::max(Mc, bp.M);
-    const size_t staged = size_t(NumLags(bits, bp.f)) * bp.R;
-    const size_t rest = (size_t(bp.f) * bp.R + kThreads) * sizeof(double2);
-    lbt = std::max(lbt, staged * sizeof(double2) + rest);
-    lbt32 = std::max(lbt32, ((staged + 1) & ~size_t(1)) * sizeof(float2) + rest);
+    const int32_t nlam = NumLags(bits, bp.f);
+    lbt = std::max(lbt, TileLds(bp, nlam, sizeof(double2)));
+    lbt32 = std::max(lbt32, TileLds(bp, nlam, sizeof(float2)));
     if (bp.logM <= kMaxLogM) {
       small = true;
       // k_bin_fft: M <= 1024 array + M/2 twiddles; larger M the padded

@@ -50,6 +50,9 @@ constexpr int kPrepBlocks = 16;    // k_bin_time workgroups computing mode terms
 constexpr int kMaxBins = 32767;    // largest B (2B-1 <= 2^kMaxLogMBig)
 constexpr int kSmallTileB = 256;   // below it a B takes the narrow class's tile width
 constexpr int kTargetTiles = 512;  // k_bin_time tiles aimed for per trial
+constexpr int kSortLogBuckets = 8;  // k_bin_time's lag sort: buckets of x
+constexpr int kSortBuckets = 1 << kSortLogBuckets;
+constexpr int kSortMaxLags = 4 * kThreads;
 constexpr int kColSlices = 4;      // k_identify holds trials*rows <= 256 entries per bin
 constexpr int kMaxTrials = 15;     // trials per iteration (odd)
 
@@ -58,6 +61,8 @@ constexpr int kMaxTrials = 15;     // trials per iteration (odd)
 struct BParams {
   int32_t B, P, f, bits, M, logM;
   int32_t R;        // residues per k_bin_time tile
+  int32_t G;        // residues that share the split of their sums (any R adds alike)
+  int32_t sorted;   // 1: the tiles visit their lags in x's order (batched form)
   int32_t slices;   // 1, or kSlices: the gather-fold split by eighths of x (one per XCD)
   int32_t slice_shift;  // log2(n) - 3 when slices > 1
   int64_t off;      // offset (in double2) of [chirp(B) | filter(M)] in table
@@ -112,7 +117,7 @@ struct IterParams {
   double width, sigma_f, dfreq;  // window (src/window.cc:28-50)
   double bin_thr, sv_thr;
   int32_t B, bits, rows, f, P, p2, M, logM, R;
-  int32_t slices, slice_shift;  // as BParams
+  int32_t G, sorted, slices, slice_shift;  // as BParams
   int32_t it;    // iteration index
   int32_t done;  // the loop stopped before this iteration
 };
@@ -135,12 +140,15 @@ struct LoopCounters {
   int32_t pad;
 };
 
-// Device-resident loop state.
-struct DevState {
+// The part of the loop state that is fixed for a call.
+struct DevFixed {
   const void *x;  // input signal (double2 or float2)
-  // fixed for a call
   int32_t mode, trials, k, min_bins, max_stale, max_iter, bits_override, B_fixed;
   double win_thr, bin_thr_fixed, sv_thr_fixed;
+};
+
+// Device-resident loop state.
+struct DevState : DevFixed {
   // updated during a call
   int32_t count;          // number of distinct found keys
   int32_t flags;
@@ -386,6 +394,9 @@ class Engine {
   // k_bin_time tiles aimed for per trial by the default tile width: fewer
   // (wider tiles) when many signals share the launches of a batch
   int32_t tile_target_ = kTargetTiles;
+  int32_t batch_count_ = 1;  // signals of the batch this engine is part of
+  // R, G, sorted and the slices of B's tiles (nlam lags).
+  void SetTile(BParams *bp, int32_t nlam) const;
 
   // recorded solve
   bool record_ = false;

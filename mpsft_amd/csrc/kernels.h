@@ -87,6 +87,7 @@ struct BatchLaunch {
   int32_t *counters;                    // device {iterations started, signals stopped}
   int32_t *host;                        // host-mapped: the counters, then the iteration's
                                         // large-path bin-FFT units
+  int32_t xcd_order;                    // gather-fold units in XCD order (k_bin_time_batch)
   int mixed;
   int large_fft = 1;                    // 0: the large-path bin-FFT launch is left out
 };

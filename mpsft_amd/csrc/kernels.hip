@@ -109,6 +109,23 @@ __device__ __forceinline__ double2 LoadX(const double2 *p) {
 }
 __device__ __forceinline__ double2 Widen(float2 v) { return make_double2(double(v.x), double(v.y)); }
 
+// A value at a wavefront-uniform address that this launch writes no byte of,
+// by scalar loads: it and what is computed from it alone stay in SGPRs.  Read
+// plainly, a batch's Ctx and IterParams (whose memory the compiler must
+// assume the kernel writes) sit in VGPRs, one copy per lane.
+typedef const uint32_t __attribute__((address_space(4))) *ConstU32;
+template <typename T>
+__device__ __forceinline__ T LoadUniform(const T *p) {
+  static_assert(sizeof(T) % 4 == 0, "read in words");
+  uint32_t w[sizeof(T) / 4];
+  const ConstU32 q = (ConstU32)p;
+#pragma unroll
+  for (size_t i = 0; i < sizeof(T) / 4; ++i) w[i] = q[i];
+  T r;
+  __builtin_memcpy(&r, w, sizeof(T));
+  return r;
+}
+
 // Window::SampleInTime (src/window.cc:71-75): w sinc(pi t w) e^{-2 (pi t
 // sigma_f)^2}, with SincPi (src/sincos.cc:69-88) = sin(x)/x and its Taylor
 // terms near 0.  sin(pi |t| w) is evaluated as sinpi(|t| w): the same value
@@ -332,6 +349,8 @@ __device__ __forceinline__ void FillParams(IterParams *ip, const BParams &bp, in
   ip->R = bp.R;
   ip->slices = bp.slices;
   ip->slice_shift = bp.slice_shift;
+  ip->G = bp.G;
+  ip->sorted = bp.sorted;
   ip->tab_off = bp.off;
   ip->width = bp.width;
   ip->sigma_f = bp.sigma_f;
@@ -393,9 +412,14 @@ __global__ void __launch_bounds__(kThreads) k_reset(Ctx c, InitArgs a) {
 // with thresholds 3 sigma/sqrt(B), sigma/sqrt(B), and the iteration's
 // transform and q's.  Reads only state that no kernel of this iteration
 // writes before k_bin_time ends, so every workgroup computes the same.
-__device__ void NextIteration(const Ctx &c, int p, IterParams *ip, LoopCounters *lc) {
+// What it reads, it reads up front and by scalar loads: a launch of a solve is
+// a few us long, and every dependent round trip at its start is in it.
+__device__ __forceinline__ void NextIteration(const Ctx &c, const DevFixed &fx, int p,
+                                              IterParams *ip, LoopCounters *lc) {
   const DevState *st = c.st;
-  const LoopCounters prev = st->L[1 - p];
+  const LoopCounters prev = LoadUniform(&st->L[1 - p]);
+  const int32_t found = LoadUniform(&st->found_iter[1 - p]);
+  const int32_t flags = LoadUniform(&st->flags), count = LoadUniform(&st->count);
   if (prev.done) {
     *lc = prev;
     ip->done = 1;
@@ -403,32 +427,32 @@ __device__ void NextIteration(const Ctx &c, int p, IterParams *ip, LoopCounters 
     return;
   }
   lc->it = prev.it + 1;
-  lc->stale = prev.stale + (st->found_iter[1 - p] ? 0 : 1);
+  lc->stale = prev.stale + (found ? 0 : 1);
   lc->pad = 0;
-  const bool replay = st->mode == kModeReplay;  // a recorded solve's iterations, no stale stop
-  const bool done = (st->flags & kFlagOverflow) || (!replay && lc->stale >= st->max_stale) ||
-                    lc->it >= st->max_iter;
+  const bool replay = fx.mode == kModeReplay;  // a recorded solve's iterations, no stale stop
+  const bool done = (flags & kFlagOverflow) || (!replay && lc->stale >= fx.max_stale) ||
+                    lc->it >= fx.max_iter;
   lc->done = done ? 1 : 0;
   ip->done = lc->done;
   ip->it = lc->it;
   if (done) return;
-  int32_t B = st->B_fixed;
-  if (st->mode == kModeSolve) {
-    const int64_t want = (int64_t(st->k) - int64_t(st->count)) * 2 + 1;
-    B = int32_t(want > st->min_bins ? want : st->min_bins);
+  int32_t B = fx.B_fixed;
+  if (fx.mode == kModeSolve) {
+    const int64_t want = (int64_t(fx.k) - int64_t(count)) * 2 + 1;
+    B = int32_t(want > fx.min_bins ? want : fx.min_bins);
   } else if (replay) {
-    B = c.log[lc->it];  // the recorded solve's bins
+    B = LoadUniform(&c.log[lc->it]);  // the recorded solve's bins
   }
-  const BParams bp = c.btab[B];
-  FillParams(ip, bp, st->bits_override > 0 ? st->bits_override : bp.bits);
-  if (st->mode == kModeSolve) {
+  const BParams bp = LoadUniform(&c.btab[B]);
+  FillParams(ip, bp, fx.bits_override > 0 ? fx.bits_override : bp.bits);
+  if (fx.mode == kModeSolve) {
     ip->bin_thr = bp.bin_thr;
     ip->sv_thr = bp.sv_thr;
   } else {
-    ip->bin_thr = st->bin_thr_fixed;
-    ip->sv_thr = st->sv_thr_fixed;
+    ip->bin_thr = fx.bin_thr_fixed;
+    ip->sv_thr = fx.sv_thr_fixed;
   }
-  ip->tf = c.tfs[lc->it];
+  ip->tf = LoadUniform(&c.tfs[lc->it]);
   // ip->q is filled by PublishIteration only: workgroups load the q of
   // their own trial, keeping the struct out of private memory.
 }
@@ -522,16 +546,16 @@ struct Lags {
     nlam = len0 + 2 * (bits - K) * f;
   }
   // lambda of staged index li
-  __device__ __forceinline__ int64_t Lambda(int li) const {
+  // (below 2^30 in magnitude: bits <= 30)
+  __device__ __forceinline__ int32_t Lambda(int li) const {
     if (li < len0) return K ? li - (1 << (K - 1)) : li;
     const int h = li - len0;
     // h / f through the float reciprocal, corrected to the exact quotient
     int seg = int(float(h) * inv_f);
     if ((seg + 1) * f <= h) ++seg;
     else if (seg * f > h) --seg;
-    const int kk = K + seg / 2;
-    const int64_t lo = (seg & 1) ? -(int64_t(1) << kk) : (int64_t(1) << kk);
-    return lo + (h - seg * f);
+    const int lo = 1 << (K + seg / 2);
+    return ((seg & 1) ? -lo : lo) + (h - seg * f);
   }
   // staged index of the first lag of row `row`
   __device__ __forceinline__ int RowStart(int row) const {
@@ -552,6 +576,24 @@ struct Lags {
 //   phase A gathers the nlam x R distinct samples into LDS (each once),
 //   phase T computes the f x R taps into LDS (each once per iteration),
 //   phase B forms every (row, rho) sum, split over `parts` threads.
+// Bound by phase A: 64 signals of n = 2^22, B = 2001 take 1144 us, 275 us
+// without the gather, and 1190 us with nothing else.  A sample is a 128-byte
+// line request, at most 62 G/s where lines miss the L2 and 227 G/s where
+// they hit, so what helps is meeting a line again while the L2 holds it:
+//  - XCD order (k_bin_time_batch): each XCD takes a contiguous range of a batch's
+//    units, so the tiles of one signal run on one L2 together;
+//  - sorted order (ip.sorted, batched signals larger than the L2s): each
+//    tile visits its lags by increasing sample position, all tiles of an
+//    XCD sweeping x alike.  Position is a B lambda mod n plus a constant of
+//    the residue, so one bucket sort of the lags serves every residue, each
+//    starting at its own bucket; R = 8 keeps 24 residues per CU resident.
+//    64 signals of n = 2^22, complex64, us per launch before / XCD order /
+//    both: B = 2001 1144 / 1056 / 952, 777 537 / 479 / 418, 311 268 / 247 /
+//    240, 101 127 / 114 / 123.  32 of n = 2^20 (8 MB each), B = 201: 73 /
+//    50 / 51.  A signal alone gains nothing from either (its x is read by
+//    all XCDs): 24.3 / 24.9 / 24.2 us at B = 2001.
+// Whatever the tile's width, a residue's sum is split and added as the
+// group of G residues it belongs to says, so results do not depend on R.
 // With ip.slices = kSlices the tile is split over the 8 XCDs: its unit s
 // gathers only the samples in the s-th eighth of x (index >> slice_shift ==
 // s; the others read as 0) and writes partial fold s.  Units go to XCDs
@@ -563,7 +605,7 @@ struct Lags {
 // found mode for this iteration.
 // blk: this workgroup's block index within the signal's launch.
 // x, qs: the signal and the iteration's q per trial.
-template <typename Tx, bool kNt = true>
+template <typename Tx, bool kNt = true, bool kSort = false>
 __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, const void *xv,
                                          const int64_t *qs, int32_t trials, int32_t tile,
                                          double2 *lds);
@@ -628,23 +670,69 @@ __device__ __forceinline__ const int64_t *IterQs(const Ctx &c, int32_t it) {
 
 template <typename Tx>
 __device__ __forceinline__ void BinTimeBody(const Ctx &c, int p, int blk, double2 *lds) {
-  const DevState *st = c.st;
+  const DevFixed fx = LoadUniform(static_cast<const DevFixed *>(c.st));
   IterParams ip;
   LoopCounters lc;
-  NextIteration(c, p, &ip, &lc);
+  NextIteration(c, fx, p, &ip, &lc);
   if (blk == 0 && threadIdx.x == 0) PublishIteration(c, p, ip, lc);
   if (ip.done) return;
-  const int32_t trials = st->trials;
   const int64_t *qs = IterQs(c, ip.it);
   if (blk < kPrepBlocks)
-    FreqTerms(c, ip, qs, trials, blk, kPrepBlocks);
+    FreqTerms(c, ip, qs, fx.trials, blk, kPrepBlocks);
   else
-    TileFold<Tx>(c, ip, st->x, qs, trials, blk - kPrepBlocks, lds);
+    TileFold<Tx>(c, ip, fx.x, qs, fx.trials, blk - kPrepBlocks, lds);
+}
+
+// The lags of a tile in buckets of increasing position a B lambda mod n (n =
+// 2^k): order[0..nlam) lists them, first[b] is where bucket b starts.  cnt:
+// kSortBuckets words of LDS free until the return.  Positions within a
+// bucket (n / 256) keep no order.
+__device__ __forceinline__ void SortLags(const Lags &L, uint32_t aB, uint32_t m32, int shift,
+                                         uint32_t *cnt, uint16_t *order, uint16_t *first) {
+  constexpr int kPer = kSortMaxLags / kThreads;
+  for (int i = threadIdx.x; i < kSortBuckets; i += kThreads) cnt[i] = 0;
+  __syncthreads();
+  uint32_t slot[kPer];  // bucket and rank within it
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int li = threadIdx.x + k * kThreads;
+    slot[k] = 0;
+    if (li < L.nlam) {
+      const uint32_t b = ((aB * uint32_t(L.Lambda(li))) & m32) >> shift;
+      slot[k] = b << 16 | atomicAdd(&cnt[b], 1u);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {  // exclusive scan of the counts by the first wavefront
+    constexpr int kQ = kSortBuckets / 64;
+    const int lane = threadIdx.x;
+    int v[kQ], sum = 0;
+#pragma unroll
+    for (int z = 0; z < kQ; ++z) {
+      v[z] = sum;
+      sum += int(cnt[lane * kQ + z]);
+    }
+    int inc = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int t = __shfl(inc, lane - d);
+      if (lane >= d) inc += t;
+    }
+#pragma unroll
+    for (int z = 0; z < kQ; ++z) first[lane * kQ + z] = uint16_t(inc - sum + v[z]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int li = threadIdx.x + k * kThreads;
+    if (li < L.nlam) order[first[slot[k] >> 16] + (slot[k] & 0xffffu)] = uint16_t(li);
+  }
+  __syncthreads();
 }
 
 // The gather-fold of one tile (trial, block of R residues) of an iteration
-// with parameters ip (see BinTimeBody).
-template <typename Tx, bool kNt>
+// with parameters ip (see BinTimeBody).  kSort: the sorted order is compiled
+// in (and taken where ip.sorted is set).
+template <typename Tx, bool kNt, bool kSort>
 __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, const void *xv,
                                          const int64_t *qs, int32_t trials, int32_t tile,
                                          double2 *lds) {
@@ -661,12 +749,13 @@ __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, con
   const int32_t rho0 = (tile - trial * nblk) * R;
   const int32_t nrho = min(R, B - rho0);
   const Lags L(bits, f);
-  const int64_t q = qs[trial];
+  const int64_t q = LoadUniform(qs + trial);
   const Tx *x = static_cast<const Tx *>(xv);
 
   // [nlam][R] samples as stored in x (complex64 samples take half the LDS
-  // and widen exactly at use), then [f][R] taps and [kThreads] partial sums
-  // in double2 (16-byte aligned).
+  // and widen exactly at use), then [f][R] taps in double2 (16-byte
+  // aligned), then the sorted order's lists and, when they are done with, the
+  // partial sums.
   Tx *X = reinterpret_cast<Tx *>(lds);
   const int xs = sizeof(Tx) == sizeof(double2) ? L.nlam * R : (L.nlam * R + 1) & ~1;
   double2 *T = reinterpret_cast<double2 *>(X + xs);
@@ -674,81 +763,125 @@ __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, con
 
   // Phase A: gather every distinct sample of the tile once, and phase T:
   // the taps tap(t), t = k*B + rho - p2 (Window::SampleInTime and the phase
-  // of src/binner.cc:100-104 with tau factored out).  Each thread issues
-  // the loads of up to kGather samples into registers, computes its taps
-  // while they are in flight, and only then writes the samples to LDS;
-  // storing each sample as it arrives would serialise the loads.
+  // of src/binner.cc:100-104 with tau factored out).  A thread keeps one
+  // residue (R divides the workgroup).  It issues the loads of up to kGather
+  // samples into registers and only then writes them to LDS; storing each
+  // sample as it arrives would serialise the loads.  One signal's launch has
+  // a workgroup or two per CU: it computes the taps while its loads are in
+  // flight.  The batched form computes them after the gather: other
+  // workgroups keep the memory system busy, and no sample's register is live
+  // across the transcendentals (three workgroups per CU).
   constexpr int kGather = 8;
   const int logR = R == 1 ? 0 : R == 2 ? 1 : R == 4 ? 2 : 3;
   const int total = L.nlam << logR;
-  const int64_t ubase = q - p2 + rho0;
-  for (int base = 0; base < total; base += kGather * kThreads) {
-    Tx g[kGather];
-#pragma unroll
-    for (int k = 0; k < kGather; ++k) {
-      const int idx = base + int(threadIdx.x) + k * kThreads;
-      const int li = idx >> logR, ri = idx & (R - 1);
-      g[k] = Tx{};
-      if (idx < total && ri < nrho) {
-        const int64_t u = ubase + L.Lambda(li) * B + ri;
-        const int64_t j = ModN(tf.a * u + tf.c, n, mask);
-        if (S == 1 || int32_t(j >> ip.slice_shift) == slice) g[k] = LoadX<kNt>(x + j);
-      }
-    }
-    if (base == 0) {
-      const double width = ip.width, sigma_f = ip.sigma_f;
-      const double delta = -0.5 / double(B);
-      for (int idx = threadIdx.x; idx < (f << logR); idx += blockDim.x) {
-        const int k = idx >> logR;
-        const int ri = idx & (R - 1);
-        if (ri < nrho) {
-          const int64_t t = int64_t(k) * B + rho0 + ri - p2;
-          // the caller's tap table is indexed as Window::wt() (t < 0 at t + P)
-          const double w = c.wtab ? c.wtab[t >= 0 ? t : t + ip.P]
-                                  : (t == 0) ? width : SampleInTime(t, width, sigma_f);
-          const int64_t r = ModN(tf.b * t, n, mask);
-          const double d = delta * double(t);
-          const double turns = double(r) / double(n) + (d - floor(d));
-          T[idx] = Scale(CisTurns(turns), w);
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kGather; ++k) {
-      const int idx = base + int(threadIdx.x) + k * kThreads;
-      if (idx < total && (idx & (R - 1)) < nrho) X[idx] = g[k];
+  const int ri = threadIdx.x & (R - 1);
+  const int64_t u0 = q - p2 + rho0 + ri;
+  // Sample of lag lambda: (a (u0 + lambda B) + c) mod n; for n = 2^k (at
+  // most 2^30) the low bits of 32-bit products.
+  const uint32_t m32 = uint32_t(mask);
+  const uint32_t aB = uint32_t(tf.a) * uint32_t(B);
+  const uint32_t s32 = uint32_t(tf.a) * uint32_t(u0) + uint32_t(tf.c);
+  const uint16_t *order = nullptr;
+  int pos = threadIdx.x >> logR;  // position in the (sorted) lag list
+  if constexpr (kSort) {
+    if (ip.sorted) {
+      uint16_t *ord = reinterpret_cast<uint16_t *>(red);
+      uint16_t *first = ord + ((L.nlam + 1) & ~1);
+      const int shift = (32 - __clz(int(m32))) - kSortLogBuckets;
+      SortLags(L, aB, m32, shift, reinterpret_cast<uint32_t *>(X), ord, first);
+      order = ord;
+      // the residue's sweep starts at sample 0: a B lambda = -s32
+      pos += first[((0u - s32) & m32) >> shift];
+      if (pos >= L.nlam) pos -= L.nlam;
     }
   }
+  auto taps = [&]() {
+    if (ri >= nrho) return;
+    const double width = ip.width, sigma_f = ip.sigma_f;
+    const double delta = -0.5 / double(B);
+    for (int idx = threadIdx.x; idx < (f << logR); idx += kThreads) {
+      const int64_t t = int64_t(idx >> logR) * B + rho0 + ri - p2;
+      // the caller's tap table is indexed as Window::wt() (t < 0 at t + P)
+      const double w = c.wtab ? c.wtab[t >= 0 ? t : t + ip.P]
+                              : (t == 0) ? width : SampleInTime(t, width, sigma_f);
+      const int64_t r = ModN(tf.b * t, n, mask);
+      const double d = delta * double(t);
+      const double turns = double(r) / double(n) + (d - floor(d));
+      T[idx] = Scale(CisTurns(turns), w);
+    }
+  };
+  for (int base = 0; base < total; base += kGather * kThreads) {
+    Tx g[kGather];
+    int put = pos;  // the same positions again, when the samples are stored
+#pragma unroll
+    for (int k = 0; k < kGather; ++k) {
+      g[k] = Tx{};
+      if (base + int(threadIdx.x) + k * kThreads < total && ri < nrho) {
+        const int li = kSort && order ? order[pos] : pos;
+        const int32_t lam = L.Lambda(li);
+        const int64_t j = mask >= 0 ? int64_t((aB * uint32_t(lam) + s32) & m32)
+                                    : ModN(tf.a * (u0 + int64_t(lam) * B) + tf.c, n, mask);
+        if (S == 1 || int32_t(j >> ip.slice_shift) == slice) g[k] = LoadX<kNt>(x + j);
+      }
+      pos += kThreads >> logR;
+      if (kSort && order && pos >= L.nlam) pos -= L.nlam;
+    }
+    if (!kSort && base == 0) taps();
+#pragma unroll
+    for (int k = 0; k < kGather; ++k) {
+      if (base + int(threadIdx.x) + k * kThreads < total && ri < nrho)
+        X[((kSort && order ? order[put] : put) << logR) + ri] = g[k];
+      put += kThreads >> logR;
+      if (kSort && order && put >= L.nlam) put -= L.nlam;
+    }
+  }
+  if constexpr (kSort) taps();
   __syncthreads();
 
-  // Phase B: per (row, rho) sums over k, split in `parts` when pairs are few.
+  // Phase B: per (row, rho) sums over k, split in `parts` threads by the
+  // size of the residue's group: G residues, or the B mod G left at the end.
+  const int32_t G = ip.G;
+  const int32_t tail0 = B - B % G;  // first residue of the short last group
+  auto parts_for = [&](int32_t width) {
+    int32_t parts = 1;
+    while (parts * 2 * rows * width <= kThreads && parts * 2 <= f) parts *= 2;
+    return parts;
+  };
+  const int32_t parts_g = parts_for(G);
+  const int32_t parts_t = tail0 < B ? parts_for(B - tail0) : parts_g;  // >= parts_g
+  const int32_t parts = rho0 + nrho > tail0 ? parts_t : parts_g;       // lanes per pair
   const int32_t pairs = rows * nrho;
-  int32_t parts = 1;
-  while (parts * 2 * pairs <= kThreads && parts * 2 <= f) parts *= 2;
   const int32_t h = (B - 1) / 2;
   double2 *fold_t = c.fold + slice * c.fold_stride + int64_t(trial) * c.rows_cap * c.B_cap;
-  for (int base = 0; base < pairs * parts; base += blockDim.x) {
+  for (int base = 0; base < pairs * parts; base += kThreads) {
     const int p = base + threadIdx.x;
     const int pair = p / parts;
     const int part = p - pair * parts;
     double2 acc = make_double2(0.0, 0.0);
-    int row = 0, ri = 0;
+    int row = 0, rj = 0, mine = 1;
     if (pair < pairs) {
       row = pair / nrho;
-      ri = pair - row * nrho;
+      rj = pair - row * nrho;
+      mine = rho0 + rj >= tail0 ? parts_t : parts_g;
       const int s0 = L.RowStart(row);
-      for (int k = part; k < f; k += parts)
-        acc = Add(acc, Cmul(Widen(X[(s0 + k) * R + ri]), T[k * R + ri]));
+      if (part < mine)
+        for (int k = part; k < f; k += mine)
+          acc = Add(acc, Cmul(Widen(X[(s0 + k) * R + rj]), T[k * R + rj]));
     }
-    if (parts > 1) {
+    // a pair's parts sit in consecutive lanes (parts is a power of two) and
+    // are added in order, two by a shuffle and more through LDS
+    if (parts == 2) {
+      const double ox = __shfl_xor(acc.x, 1), oy = __shfl_xor(acc.y, 1);
+      if (mine == 2) acc = Add(acc, make_double2(ox, oy));
+    } else if (parts > 2) {
       red[threadIdx.x] = acc;
       __syncthreads();
-      if (pair < pairs && part == 0)
-        for (int j = 1; j < parts; ++j) acc = Add(acc, red[threadIdx.x + j]);
+      if (part == 0)
+        for (int j = 1; j < mine; ++j) acc = Add(acc, red[threadIdx.x + j]);
       __syncthreads();
     }
     if (pair < pairs && part == 0) {
-      const int rho = rho0 + ri;
+      const int rho = rho0 + rj;
       const int m = rho >= h ? rho - h : rho - h + B;
       fold_t[int64_t(row) * c.B_cap + m] = acc;
     }
@@ -1827,17 +1960,17 @@ inline int ColSlicesFor(int64_t trials_rows) { return trials_rows <= 64 ? 1 : kC
 // at the start of the iteration of parity p.
 
 // Iteration parameters of a late iteration (false: it does not exist).
-__device__ __forceinline__ bool LateGeometry(const Ctx &c, int p, IterParams *ip) {
-  const DevState *st = c.st;
-  const LoopCounters prev = st->L[1 - p];
+__device__ __forceinline__ bool LateGeometry(const Ctx &c, const DevFixed &fx, int p,
+                                             IterParams *ip) {
+  const LoopCounters prev = LoadUniform(&c.st->L[1 - p]);
   if (prev.done) return false;
   const int32_t it = prev.it + 1;
-  if (it >= st->max_iter) return false;
-  const BParams bp = c.btab[st->min_bins];
+  if (it >= fx.max_iter) return false;
+  const BParams bp = LoadUniform(&c.btab[fx.min_bins]);
   FillParams(ip, bp, bp.bits);
   ip->bin_thr = bp.bin_thr;
   ip->sv_thr = bp.sv_thr;
-  ip->tf = c.tfs[it];
+  ip->tf = LoadUniform(&c.tfs[it]);
   ip->it = it;
   ip->done = 0;
   return true;
@@ -1861,10 +1994,11 @@ __global__ void __launch_bounds__(kThreads)
     if (with_identify) IdentifyBody<NS, false>(c, 1 - p, blk, nb_ident);
     return;
   }
+  const DevFixed fx = LoadUniform(static_cast<const DevFixed *>(c.st));
   IterParams ip;
-  if (!LateGeometry(c, p, &ip)) return;
+  if (!LateGeometry(c, fx, p, &ip)) return;
   DevState *st = c.st;
-  const int32_t trials = st->trials;
+  const int32_t trials = fx.trials;
   const int32_t pb = blk - nb_ident;
   if (pb == 0 && threadIdx.x == 0) {  // publish the geometry for k_late_fft
     st->P[p] = ip;
@@ -1899,7 +2033,7 @@ __global__ void __launch_bounds__(kThreads)
     }
     return;
   }
-  TileFold<Tx>(c, ip, st->x, IterQs(c, ip.it), trials, pb - kPrepBlocks, lds);
+  TileFold<Tx>(c, ip, fx.x, IterQs(c, ip.it), trials, pb - kPrepBlocks, lds);
 }
 
 template <int kPaths>
@@ -2213,8 +2347,9 @@ __global__ void __launch_bounds__(64)
   const Ctx &c = ctxs[i];
   // the iteration's parameters are built in place, in slot p
   IterParams &ip = c.st->P[p];
+  const DevFixed fx = LoadUniform(static_cast<const DevFixed *>(c.st));
   LoopCounters lc;
-  NextIteration(c, p, &ip, &lc);
+  NextIteration(c, fx, p, &ip, &lc);
   PublishLoop(c, p, ip, lc);
   int32_t u[kUnitKinds] = {0, 0, 0, 0};
   if (!ip.done) {
@@ -2342,25 +2477,33 @@ __global__ void __launch_bounds__(kPlanThreads)
 template <typename Tx>
 __device__ __forceinline__ void BinTimeUnit(const Ctx &c, int p, int32_t unit, double2 *lds) {
   const DevState *st = c.st;
-  const IterParams &ip = st->P[p];
-  const int32_t trials = st->trials;
+  const IterParams ip = LoadUniform(&st->P[p]);
+  const int32_t trials = LoadUniform(&st->trials);
   const int64_t *qs = IterQs(c, ip.it);
-  const int32_t nprep = PrepUnits(int64_t(min(st->count, c.cap)) * trials);
+  const int32_t nprep = PrepUnits(int64_t(min(LoadUniform(&st->count), c.cap)) * trials);
   if (unit < nprep)
     FreqTerms(c, ip, qs, trials, unit, nprep);
   else
-    TileFold<Tx, false>(c, ip, st->x, qs, trials, unit - nprep, lds);
+    TileFold<Tx, false, true>(c, ip, LoadUniform(&st->x), qs, trials, unit - nprep, lds);
 }
 
 template <typename Tx>
-__global__ void __launch_bounds__(kThreads)
-    k_bin_time_batch(const Ctx *ctxs, const int2 *map, const int32_t *total, int p) {
+__global__ void __launch_bounds__(kThreads, 3)
+    k_bin_time_batch(const Ctx *ctxs, const int2 *map, const int32_t *total, int32_t xcd_order,
+                     int p) {
   HIP_DYNAMIC_SHARED(double2, lds)
-  const int32_t tot = total[0];
-  for (int32_t u = blockIdx.x; u < tot; u += gridDim.x) {
-    if (u != int32_t(blockIdx.x)) __syncthreads();  // the previous unit's LDS reads are done
-    const int2 m = map[u];
-    BinTimeUnit<Tx>(ctxs[m.x], p, m.y, lds);
+  const int32_t tot = LoadUniform(total);
+  // Workgroups go to the 8 XCDs round robin.  XCD order: XCD i takes the
+  // i-th eighth of the units, so that the tiles of a signal, consecutive in
+  // the map, meet in one L2.
+  const int32_t per = xcd_order ? (tot + 7) / 8 : tot;
+  const int32_t step = xcd_order ? gridDim.x / 8 : gridDim.x;
+  const int32_t first = xcd_order ? blockIdx.x / 8 : blockIdx.x;
+  const int32_t u0 = xcd_order ? (blockIdx.x % 8) * per : 0;
+  for (int32_t i = first; i < per && u0 + i < tot; i += step) {
+    if (i != first) __syncthreads();  // the previous unit's LDS reads are done
+    const int2 m = LoadUniform(map + u0 + i);
+    BinTimeUnit<Tx>(LoadUniform(ctxs + m.x), p, m.y, lds);
   }
 }
 
@@ -3178,10 +3321,10 @@ hipError_t LaunchBatchStage(const BatchLaunch &b, int parity, int stage, hipStre
     case 1:
       if (b.mixed)
         hipLaunchKernelGGL(k_bin_time_batch<float2>, dim3(b.grid_time), dim3(kThreads),
-                           b.lds_time, s, b.ctxs, w.map[0], w.total, parity);
+                           b.lds_time, s, b.ctxs, w.map[0], w.total, b.xcd_order, parity);
       else
         hipLaunchKernelGGL(k_bin_time_batch<double2>, dim3(b.grid_time), dim3(kThreads),
-                           b.lds_time, s, b.ctxs, w.map[0], w.total, parity);
+                           b.lds_time, s, b.ctxs, w.map[0], w.total, b.xcd_order, parity);
       break;
     case 2:  // one kernel per bin-FFT path, each over its own units
       hipLaunchKernelGGL(k_bin_fft_batch<kFftSmallOnly>, dim3(b.grid_fft), dim3(kFftThreads),

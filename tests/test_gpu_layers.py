@@ -52,3 +52,38 @@ def test_iterate_after_overflow_changes_nothing(gpu):
         got = s.modes_dict()
         assert len(got) == 4 and (rep == 0 or got == first)
         first = got
+
+
+@pytest.mark.parametrize("n,ks,precision,trials", [
+    # first bins 2 k + 1 on both sides of the sorted order's 256; ragged last
+    # tiles (B mod 8 = 1 .. 7) and wide ones (8 residues); three trials
+    (1 << 20, (127, 128), "FP64", 1), (1 << 21, (600, 303, 140), "MIXED", 1),
+    (1 << 21, (150, 130, 129, 131), "MIXED", 3), (1 << 20, (500, 451), "FP64", 3)])
+def test_batch_sorted_tiles_match_single(gpu, n, ks, precision, trials):
+    """Signals of 16 MB and more take the sorted gather order in a batch
+    (and XCD order); a signal alone takes neither.  Same decisions, and
+    coefficients to rounding (the sums are split differently)."""
+    from mpsft_amd.signals import make_signal, quantization_sigma
+    prec = gpu.MPSFT_FP64 if precision == "FP64" else gpu.MPSFT_MIXED
+    xs, opts = [], []
+    for i, k in enumerate(ks):
+        x, _ = make_signal(n, k, 1e-6, seed=50 + i)
+        sig = 1e-6
+        if precision == "MIXED":
+            x64 = x.astype(np.complex64)
+            sig = float(np.hypot(sig, quantization_sigma(x, x64)))
+            x = x64
+        xs.append(x)
+        opts.append(gpu.solve_options(k, sig, trials=trials))
+    seeds = [9 + i for i in range(len(ks))]
+    batch = gpu.Batch([n] * len(ks), opts, prec)
+    iters, status = batch.solve(batch.upload(xs), seeds)
+    assert all(v == 0 for v in status)
+    for i, x in enumerate(xs):
+        s = gpu.Solver(n, opts[i], prec)
+        assert s.solve(s.upload(x), seeds[i]) == iters[i]
+        want, got = s.modes_dict(), batch.modes_dict(i)
+        assert set(got) == set(want)
+        top = max(abs(v) for v in want.values())
+        for key, v in want.items():
+            assert abs(got[key] - v) <= TOL * max(abs(v), 1e-2 * top)
