@@ -115,6 +115,12 @@ size_t TileLds(const BParams &bp, int32_t nlam, size_t elem) {
          (size_t(bp.f) * bp.R + kThreads) * sizeof(double2);
 }
 
+// LDS of one k_bin_fft workgroup (B <= kMaxLdsBins).
+size_t FftLds(const BParams &bp) {
+  if (bp.B <= kDirectBins) return kDirectLds;
+  return size_t(bp.logM <= kFftSmallLogM ? bp.M + bp.M / 2 : bp.M + bp.M / 16) * sizeof(double2);
+}
+
 // Transforms drawn before a solve's first launch.
 constexpr int32_t kFirstDraws = 32;
 
@@ -440,7 +446,7 @@ int Engine::EnsureTables(const std::vector<int32_t> &bs, double delta, int32_t b
     bp.off = 0;
     if (bp.logM <= kMaxLogM) {
       bp.off = table_used_ + need;
-      need += B + bp.M;
+      need += B <= kDirectBins ? B : B + bp.M;
       todo.push_back(B);
       Mmax = std::max(Mmax, bp.M);
     }
@@ -549,13 +555,12 @@ int Engine::Reserve(int32_t trials, const std::vector<int32_t> &bs) {
     lbt32 = std::max(lbt32, TileLds(bp, nlam, sizeof(float2)));
     if (bp.logM <= kMaxLogM) {
       small = true;
-      // k_bin_fft: M <= 1024 array + M/2 twiddles; larger M the padded
-      // array (M + M/16).  The BinInFreq limbs of the B bins (four 8-byte
+      // k_bin_fft: the direct DFT's arrays; M = 1024 array + M/2 twiddles;
+      // larger M the padded array (M + M/16).  The BinInFreq limbs of the B bins (four 8-byte
       // integers per bin: 2B <= M double2 slots) later take the array's place.
-      const size_t el = bp.logM <= kFftSmallLogM ? size_t(bp.M + bp.M / 2)
-                                                 : size_t(bp.M + bp.M / 16);
-      lfft = std::max(lfft, el * sizeof(double2));
-      if (bp.logM <= kFftSmallLogM) lfft_small = std::max(lfft_small, el * sizeof(double2));
+      const size_t bytes = FftLds(bp);
+      lfft = std::max(lfft, bytes);
+      if (bp.logM <= kFftSmallLogM) lfft_small = std::max(lfft_small, bytes);
     } else {
       big = true;
       Mbig = std::max(Mbig, bp.M);
@@ -808,9 +813,9 @@ int Engine::EnsureGraph(int32_t iters, hipStream_t s) {
     const int32_t nb_ident = std::max<int32_t>(1, (late_B_ + waves - 1) / waves);
     const int32_t tiles = trials_cap_ * ((late_B_ + bp.R - 1) / bp.R) * bp.slices;
     // the late B's bin FFT on its own path: the small one's kernel and LDS
-    // (array M and M/2 twiddles) where it applies
+    // where it applies
     const bool small_fft = bp.logM <= kFftSmallLogM;
-    const size_t lds_fft = small_fft ? size_t(bp.M + bp.M / 2) * sizeof(double2) : LdsFft();
+    const size_t lds_fft = small_fft ? FftLds(bp) : LdsFft();
     for (int k = 2; k < 4; ++k) {
       hipStream_t cs;
       HIP_OK(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));

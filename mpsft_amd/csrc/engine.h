@@ -41,6 +41,8 @@ constexpr int kFftThreads = 256;   // workgroup size of k_bin_fft
 constexpr int kMaxLogM = 12;       // k_bin_fft (one LDS FFT) up to M = 4096, B <= 2048
 constexpr int kMaxLdsBins = 2048;  // largest B of k_bin_fft
 constexpr int kFftSmallLogM = 10;  // k_bin_fft's in-place radix-4 path up to M = 1024
+constexpr int kDirectBins = 255;   // largest B whose bin DFT is computed directly
+constexpr size_t kDirectLds = 16 * 1024;  // its LDS
 constexpr int kMaxLogMBig = 16;    // four-step Bluestein FFT up to M = 65536
 constexpr int kTwLogM = kMaxLogMBig;  // twiddle table e^{-2 pi i j / 2^kTwLogM}
 constexpr int kBigTile = 1024;     // elements of one four-step workgroup
@@ -65,8 +67,9 @@ struct BParams {
   int32_t sorted;   // 1: the tiles visit their lags in x's order (batched form)
   int32_t slices;   // 1, or kSlices: the gather-fold split by eighths of x (one per XCD)
   int32_t slice_shift;  // log2(n) - 3 when slices > 1
-  int64_t off;      // offset (in double2) of [chirp(B) | filter(M)] in table
-                    // (B <= kMaxLdsBins only; larger B compute both on the fly)
+  int64_t off;      // offset (in double2) of [w(B)] (B <= kDirectBins) or
+                    // [chirp(B) | filter(M)] in table (B <= kMaxLdsBins only;
+                    // larger B compute both on the fly)
   double width;     // 1/(2B)
   double sigma_f;   // window std-dev in frequency
   double dfreq;     // sqrt(2)*pi*sigma_t  (SampleInFreq)

@@ -287,8 +287,9 @@ __global__ void __launch_bounds__(kThreads) k_build_twiddles(double2 *tw) {
   }
 }
 
-// One workgroup per B: chirp c_m (m < B) and the spectrum of the Bluestein
-// filter h (h_j = conj(c_j), h_{M-j} = conj(c_j)), pre-scaled by 1/M.
+// One workgroup per B.  B <= kDirectBins: w_j = e^{-2 pi i j/B}, j < B.
+// Larger B: chirp c_m (m < B) and the spectrum of the Bluestein filter h (h_j
+// = conj(c_j), h_{M-j} = conj(c_j)), pre-scaled by 1/M.
 __global__ void __launch_bounds__(kThreads)
     k_build_tables(const int32_t *blist, const BParams *btab, double2 *table,
                    const double2 *tw) {
@@ -296,6 +297,15 @@ __global__ void __launch_bounds__(kThreads)
   const int32_t B = blist[blockIdx.x];
   const BParams bp = btab[B];
   double2 *chirp = table + bp.off;
+  if (B <= kDirectBins) {
+    for (int j = threadIdx.x; j < B; j += blockDim.x) {
+      const int r = min(j, B - j);  // at most half a turn: w_(B-j) = conj(w_j)
+      double s, c;
+      sincospi(2.0 * double(r) / double(B), &s, &c);
+      chirp[j] = make_double2(c, r == j ? -s : s);
+    }
+    return;
+  }
   double2 *filt = chirp + B;
   const int M = bp.M;
   for (int m = threadIdx.x; m < B; m += blockDim.x) chirp[m] = Chirp(m, B);
@@ -1223,7 +1233,7 @@ __device__ __forceinline__ void StoreBins(double2 *A, int32_t B, const double2 (
 // BinInFreqV1 subtraction (src/binner.cc:565-591) of every found mode
 // (terms from k_bin_time).  Every global load is issued up front.  Two
 // paths, chosen by M for the whole launch:
-//   M <= 1024 (B <= 512): in-place radix-4 passes in LDS (bit-reversed
+//   M = 1024 (257 <= B <= 511): in-place radix-4 passes in LDS (bit-reversed
 //     DIT forward, DIF inverse), twiddles staged in LDS; up to 256
 //     butterflies per pass keep every thread busy at small M;
 //   M = 2048, 4096: the register Stockham passes above, the forward
@@ -1406,14 +1416,145 @@ __device__ __forceinline__ void BinFftLarge(const Ctx &c, const IterParams &ip, 
   }
 }
 
+// ---------------------------------------------------------------------------
+// The bin DFT of B <= kDirectBins points, directly.  With e_m = x_m + x_(B-m)
+// and o_m = x_m - x_(B-m) (m = 1 .. h = (B-1)/2; B is odd), w_j =
+// e^(-2 pi i j/B):
+//   X_k     = x_0 + sum_m e_m Re w_mk + i sum_m o_m Im w_mk,
+//   X_(B-k) = x_0 + sum_m e_m Re w_mk - i sum_m o_m Im w_mk,
+// so a pair of outputs costs 4 FMAs per pair of inputs, B^2 in all, and no
+// barrier between the loads and the result; four lanes share a k and split m.
+// Bluestein's two M-point transforms (M <= 512) are eight to ten dependent
+// passes with a barrier each: 8500 of the 22000 cycles of a late iteration's
+// bin FFT at B = 101, where this takes 1500.  The per-bin BinInFreq sums do
+// not need the DFT's LDS here, so they are built beside it, between the same
+// two barriers.  Bound by the twiddle reads (one 16-byte LDS gather per pair
+// of pairs): at B = 511 they would take as long as the passes, hence the
+// limit at half of that.
+// us: a late iteration's launch at n = 2^22, S = 1000 (B = 101, 33 rows)
+// 10.4 -> 7.3; a BinInTime call at n = 2^16, B = 101 12.7 -> 11.0.  Its error
+// is the smaller: 7.3e-16 of the norm against 8.1e-16 (that call, with the
+// gather-fold's share).
+constexpr int kDirectPer = (kDirectBins / 2 + 1 + 63) / 64;  // k's per thread
+struct DirectOut {
+  double2 x[kDirectPer];
+  int32_t k[kDirectPer];  // the bin of x[i], or -1
+};
+struct DirectLds {
+  double2 e[kDirectBins / 2 + 1], o[kDirectBins / 2 + 1], w[kDirectBins];
+  unsigned long long limbs[4 * kDirectBins];
+};
+static_assert(sizeof(DirectLds) <= kDirectLds, "LDS of the direct bin DFT");
+
+// Loads of x (conjugated with CONJ_IN) and w into LDS; the caller
+// synchronises before DirectDft.
+template <bool CONJ_IN>
+__device__ __forceinline__ void DirectStage(const Ctx &c, const IterParams &ip, const double2 *fold,
+                                            DirectLds *l) {
+  const int32_t B = ip.B, h = (B - 1) / 2;
+  const int m = threadIdx.x;
+  if (m < B) l->w[m] = (c.table + ip.tab_off)[m];
+  if (m <= h) {
+    const int mb = m ? B - m : 0;
+    double2 a, b;
+    if (CONJ_IN) {
+      a = Conj(fold[m]);
+      b = Conj(fold[mb]);
+    } else {
+      a = FoldAt(fold, m, ip.slices, c.fold_stride);
+      b = FoldAt(fold, mb, ip.slices, c.fold_stride);
+    }
+    l->e[m] = m ? Add(a, b) : a;
+    l->o[m] = Sub(a, b);
+  }
+}
+
+// This thread's outputs, times rp.
+__device__ __forceinline__ void DirectDft(int32_t B, double2 rp, const DirectLds *l, DirectOut *out) {
+  const int32_t h = (B - 1) / 2;
+  const int g = threadIdx.x & 3, slot = threadIdx.x >> 2;
+  double2 ec[kDirectPer], os[kDirectPer];
+  int idx[kDirectPer], step[kDirectPer];
+#pragma unroll
+  for (int i = 0; i < kDirectPer; ++i) {
+    const int k = min(slot + 64 * i, h);
+    ec[i] = os[i] = make_double2(0.0, 0.0);
+    idx[i] = k * (1 + g) % B;
+    step[i] = 4 * k % B;
+  }
+  const bool both = h >= 64;  // the second k of a thread exists
+  for (int m = 1 + g; m <= h; m += 4) {
+    const double2 e = l->e[m], o = l->o[m];
+#pragma unroll
+    for (int i = 0; i < kDirectPer; ++i) {
+      if (i > 0 && !both) break;
+      const double2 w = l->w[idx[i]];
+      ec[i].x = fma(e.x, w.x, ec[i].x);
+      ec[i].y = fma(e.y, w.x, ec[i].y);
+      os[i].x = fma(o.x, w.y, os[i].x);
+      os[i].y = fma(o.y, w.y, os[i].y);
+      idx[i] += step[i];
+      if (idx[i] >= B) idx[i] -= B;
+    }
+  }
+  const double2 x0 = l->e[0];
+#pragma unroll
+  for (int i = 0; i < kDirectPer; ++i) {
+    for (int d = 1; d < 4; d <<= 1) {
+      ec[i].x += __shfl_xor(ec[i].x, d);
+      ec[i].y += __shfl_xor(ec[i].y, d);
+      os[i].x += __shfl_xor(os[i].x, d);
+      os[i].y += __shfl_xor(os[i].y, d);
+    }
+    const int k = slot + 64 * i;
+    const double2 even = Add(x0, ec[i]), odd = MulPosI(os[i]);
+    out->k[i] = k > h ? -1 : g == 0 ? k : g == 1 && k > 0 ? B - k : -1;
+    out->x[i] = Cmul(g == 0 ? Add(even, odd) : Sub(even, odd), rp);
+  }
+}
+
+// DFT, row phase and BinInFreq of one row.  val, bin: this thread's first N
+// terms (modes threadIdx.x + r kFftThreads < cnt); term(i, &bin) forms any
+// later one; mx: the largest component of all the thread's terms.
+template <int N, typename Term>
+__device__ __forceinline__ void DirectRow(const Ctx &c, const IterParams &ip, const double2 *fold,
+                                          double2 rp, double2 *lds, const double2 (&val)[N],
+                                          const int (&bin)[N], int32_t cnt, double mx, Term term,
+                                          double2 *A) {
+  constexpr int T = kFftThreads;
+  DirectLds *l = reinterpret_cast<DirectLds *>(lds);
+  const int32_t B = ip.B;
+  const int tid = threadIdx.x;
+  DirectStage<false>(c, ip, fold, l);
+  for (int k = tid; k < kLimbs * B; k += T) l->limbs[k] = 0ull;
+  const TermGrid g = MakeTermGrid(mx);  // its barrier: the staged row is ready too
+  if (g.any) {
+#pragma unroll
+    for (int r = 0; r < N; ++r)
+      if (tid + r * T < cnt) LimbAdd(l->limbs + kLimbs * bin[r], val[r], g);
+    for (int i = tid + N * T; i < cnt; i += T) {
+      int32_t b;
+      const double2 v = term(i, &b);
+      LimbAdd(l->limbs + kLimbs * b, v, g);
+    }
+  }
+  DirectOut out;
+  DirectDft(B, rp, l, &out);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kDirectPer; ++i)
+    if (out.k[i] >= 0)
+      A[out.k[i]] = g.any ? Sub(out.x[i], LimbValue(l->limbs + kLimbs * out.k[i], g)) : out.x[i];
+}
+
 template <int kPaths>
 __device__ __forceinline__ void BinFftBody(const Ctx &c, int p, int blk, double2 *lds) {
   constexpr int T = kFftThreads;
   constexpr int kPerTerm = 2;  // BinInFreq terms prefetched per thread
   const DevState *st = c.st;
-  const IterParams &ip = st->P[p];
+  const IterParams ip = LoadUniform(&st->P[p]);
   if (ip.done || ip.logM > kMaxLogM || !FftPathMatches<kPaths>(ip)) return;
-  const int32_t trials = st->trials, rows = ip.rows;
+  const int32_t trials = LoadUniform(&st->trials), rows = ip.rows;
   const int32_t trial = blk / c.rows_cap;
   const int32_t row = blk - trial * c.rows_cap;
   if (trial >= trials || row >= rows) return;
@@ -1421,7 +1562,7 @@ __device__ __forceinline__ void BinFftBody(const Ctx &c, int p, int blk, double2
   const int tid = threadIdx.x;
   const int64_t n = c.n, mask = c.mask;
   const double2 *fold = c.fold + (int64_t(trial) * c.rows_cap + row) * c.B_cap;
-  const int32_t cnt = min(st->count, c.cap);
+  const int32_t cnt = min(LoadUniform(&st->count), c.cap);
   const int32_t *tb = c.term_bin + int64_t(trial) * c.cap;
   const double2 *tv = c.term_val + (int64_t(trial) * c.rows_cap + row) * c.cap;
   double2 tval[kPerTerm];
@@ -1436,8 +1577,23 @@ __device__ __forceinline__ void BinFftBody(const Ctx &c, int p, int blk, double2
       tval[r] = tv[i];
     }
   }
-  const int64_t tau = ModN(ip.q[trial] + RowOffset(row) * B, n, mask);
+  const int64_t tau = ModN(LoadUniform(&st->P[p].q[trial]) + RowOffset(row) * B, n, mask);
   const double2 rp = CisFrac(ModN(ip.tf.b * tau, n, mask), n);
+  double mx = 0.0;
+#pragma unroll
+  for (int r = 0; r < kPerTerm; ++r)
+    if (tid + r * T < cnt) mx = fmax(mx, MaxComp(tval[r]));
+  for (int i = tid + kPerTerm * T; i < cnt; i += T) mx = fmax(mx, MaxComp(tv[i]));
+  double2 *A = c.A + (int64_t(trial) * c.rows_cap + row) * c.B_cap;
+  if (kPaths != kFftLargeOnly && B <= kDirectBins) {
+    DirectRow(c, ip, fold, rp, lds, tval, tbin, cnt, mx,
+              [&](int i, int32_t *bin) {
+                *bin = tb[i];
+                return tv[i];
+              },
+              A);
+    return;
+  }
   double2 *a = lds;
   const bool small = ip.logM <= kFftSmallLogM;
   if constexpr (kPaths == kFftSmallOnly) {
@@ -1457,11 +1613,6 @@ __device__ __forceinline__ void BinFftBody(const Ctx &c, int p, int blk, double2
   double2 xo[OutPer<kPaths>()];
   TakeOutputs(a, small, B, xo);
   unsigned long long *limbs = reinterpret_cast<unsigned long long *>(a);
-  double mx = 0.0;
-#pragma unroll
-  for (int r = 0; r < kPerTerm; ++r)
-    if (tid + r * T < cnt) mx = fmax(mx, MaxComp(tval[r]));
-  for (int i = tid + kPerTerm * T; i < cnt; i += T) mx = fmax(mx, MaxComp(tv[i]));
   for (int k = tid; k < kLimbs * B; k += T) limbs[k] = 0ull;
   const TermGrid g = MakeTermGrid(mx);
   if (g.any) {
@@ -1471,7 +1622,7 @@ __device__ __forceinline__ void BinFftBody(const Ctx &c, int p, int blk, double2
     for (int i = tid + kPerTerm * T; i < cnt; i += T) LimbAdd(limbs + kLimbs * tb[i], tv[i], g);
   }
   __syncthreads();
-  StoreBins(c.A + (int64_t(trial) * c.rows_cap + row) * c.B_cap, B, xo, limbs, g);
+  StoreBins(A, B, xo, limbs, g);
 }
 
 __global__ void __launch_bounds__(kFftThreads) k_bin_fft(Ctx c, int p) {
@@ -2044,7 +2195,11 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
   DevState *st = c.st;
   // Loop control of this iteration (NextIteration's; identify of the
   // previous iteration has finished).
-  const LoopCounters prev = st->L[1 - p];
+  const LoopCounters prev = LoadUniform(&st->L[1 - p]);
+  const DevFixed fx = LoadUniform(static_cast<const DevFixed *>(st));
+  const int32_t found = LoadUniform(&st->found_iter[1 - p]);
+  const int32_t flags = LoadUniform(&st->flags), count = LoadUniform(&st->count);
+  const int32_t cnt_pre = min(LoadUniform(&st->cnt_base[1 - p]), c.cap);  // modes with factors
   if (prev.done) {
     // Past the stop: carry it into this parity's slots, so the launches
     // still queued behind this one (the next k_late_fold's identify and
@@ -2058,31 +2213,31 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
   }
   LoopCounters lc;
   lc.it = prev.it + 1;
-  lc.stale = prev.stale + (st->found_iter[1 - p] ? 0 : 1);
+  lc.stale = prev.stale + (found ? 0 : 1);
   lc.pad = 0;
   const bool done =
-      (st->flags & kFlagOverflow) || lc.stale >= st->max_stale || lc.it >= st->max_iter;
+      (flags & kFlagOverflow) || lc.stale >= fx.max_stale || lc.it >= fx.max_iter;
   lc.done = done ? 1 : 0;
-  const int32_t cnt_pre = min(st->cnt_base[1 - p], c.cap);  // modes with factors
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     // PublishIteration's bookkeeping, for the slot k_late_fold filled.
     st->L[p] = lc;
     st->P[p].done = lc.done;  // read by the next launch's identify
     st->found_iter[p] = 0;
-    st->cnt_base[p] = st->count;
-    if (st->mode == kModeSolve && prev.it >= 0 && prev.it < c.log_cap) {
+    st->cnt_base[p] = count;
+    if (fx.mode == kModeSolve && prev.it >= 0 && prev.it < c.log_cap) {
       c.log[prev.it] = st->P[1 - p].B;
-      c.log[c.log_cap + prev.it] = st->count;
+      c.log[c.log_cap + prev.it] = count;
     }
     if (lc.done) {
       st->iters = lc.it;
       st->stop_stale = lc.stale;
     }
-    if (c.progress && lc.done) PublishStop(c, lc.it, lc.stale, st->flags);
+    if (c.progress && lc.done) PublishStop(c, lc.it, lc.stale, flags);
   }
   if (done) return;
-  const IterParams &ip = st->P[p];
-  const int32_t trials = st->trials, rows = ip.rows;
+  // (the launch writes P[p].done, which is not read from here on)
+  const IterParams ip = LoadUniform(&st->P[p]);
+  const int32_t trials = fx.trials, rows = ip.rows;
   const int32_t trial = blockIdx.x / c.rows_cap;
   const int32_t row = blockIdx.x - trial * c.rows_cap;
   if (trial >= trials || row >= rows) return;
@@ -2090,7 +2245,7 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
   const int tid = threadIdx.x;
   const int64_t n = c.n, mask = c.mask;
   const double2 *fold = c.fold + (int64_t(trial) * c.rows_cap + row) * c.B_cap;
-  const int32_t cnt = min(st->count, c.cap);
+  const int32_t cnt = min(count, c.cap);
   const int32_t *tb = c.term_bin + int64_t(trial) * c.cap;
   const double2 *tv = c.term_val + (int64_t(trial) * c.rows_cap + row) * c.cap;
   // prefetch: factor, bin and key of the first modes
@@ -2109,7 +2264,7 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
       tbin[r] = tb[i];
     }
   }
-  const int64_t q = ip.q[trial];
+  const int64_t q = LoadUniform(&st->P[p].q[trial]);
   const int64_t tau = ModN(q + RowOffset(row) * B, n, mask);
   const double2 rp = CisFrac(ModN(ip.tf.b * tau, n, mask), n);
   // their coefficients, final since the previous launch (identify of the
@@ -2117,23 +2272,8 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
   double2 cfv[kPerTerm];
 #pragma unroll
   for (int r = 0; r < kPerTerm; ++r) cfv[r] = kk[r] >= 0 ? c.coef[kk[r]] : make_double2(0.0, 0.0);
-  double2 *a = lds;
-  const bool small = ip.logM <= kFftSmallLogM;
-  if constexpr (kPaths == kFftSmallOnly) {
-    BinFftSmall<false>(c, ip, fold, rp, a);
-  } else {
-    if (small)
-      BinFftSmall<false>(c, ip, fold, rp, a);
-    else
-      BinFftLarge<false>(c, ip, fold, rp, a);
-  }
-  __syncthreads();
-  // BinInFreq, as k_bin_fft's epilogue (exact per-bin sums of the terms):
-  // the terms of the first modes are formed once, in registers, and the
-  // rest (more than kPerTerm x T modes) are formed again for the second pass.
-  double2 xo[OutPer<kPaths>()];
-  TakeOutputs(a, small, B, xo);
-  unsigned long long *limbs = reinterpret_cast<unsigned long long *>(a);
+  // The terms of the first modes are formed once, in registers, and the rest
+  // (more than kPerTerm x T modes) are formed again for the second pass.
   auto term = [&](int i, int64_t k0, const double2 &cf, int32_t *bin) {
     if (i < cnt_pre) {
       *bin = tb[i];
@@ -2163,6 +2303,31 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
     const int64_t k0 = c.keys[i];
     mx = fmax(mx, MaxComp(term(i, k0, c.coef[k0], &bin)));
   }
+  double2 *A = c.A + (int64_t(trial) * c.rows_cap + row) * c.B_cap;
+  if (B <= kDirectBins) {
+    DirectRow(c, ip, fold, rp, lds, vr, tbin, cnt, mx,
+              [&](int i, int32_t *bin) {
+                const int64_t k0 = c.keys[i];
+                return term(i, k0, c.coef[k0], bin);
+              },
+              A);
+    return;
+  }
+  double2 *a = lds;
+  const bool small = ip.logM <= kFftSmallLogM;
+  if constexpr (kPaths == kFftSmallOnly) {
+    BinFftSmall<false>(c, ip, fold, rp, a);
+  } else {
+    if (small)
+      BinFftSmall<false>(c, ip, fold, rp, a);
+    else
+      BinFftLarge<false>(c, ip, fold, rp, a);
+  }
+  __syncthreads();
+  // BinInFreq, as k_bin_fft's epilogue (exact per-bin sums of the terms).
+  double2 xo[OutPer<kPaths>()];
+  TakeOutputs(a, small, B, xo);
+  unsigned long long *limbs = reinterpret_cast<unsigned long long *>(a);
   for (int k = tid; k < kLimbs * B; k += T) limbs[k] = 0ull;
   const TermGrid g = MakeTermGrid(mx);
   if (g.any) {
@@ -2177,7 +2342,7 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
     }
   }
   __syncthreads();
-  StoreBins(c.A + (int64_t(trial) * c.rows_cap + row) * c.B_cap, B, xo, limbs, g);
+  StoreBins(A, B, xo, limbs, g);
 }
 
 // BinInFreqV1 (src/binner.cc:565-591) on a caller-owned bin matrix (rows x
@@ -2662,6 +2827,17 @@ __device__ __forceinline__ void AdjFftBody(const Ctx &c, const IterParams &ip, i
   const int64_t tau = ModN(ip.q[trial] + RowOffset(row) * B, n, mask);
   const double2 rp = CisFrac(ModN(ip.tf.b * tau, n, mask), n);
   const int64_t off = (int64_t(trial) * c.rows_cap + row) * c.B_cap;
+  if (B <= kDirectBins) {
+    DirectLds *l = reinterpret_cast<DirectLds *>(lds);
+    DirectStage<true>(c, ip, c.A + off, l);
+    __syncthreads();
+    DirectOut out;
+    DirectDft(B, rp, l, &out);
+#pragma unroll
+    for (int i = 0; i < kDirectPer; ++i)
+      if (out.k[i] >= 0) fbar[off + out.k[i]] = Conj(out.x[i]);
+    return;
+  }
   double2 *a = lds;
   // kFftSmallOnly: the launch's signals all have M <= 2^kFftSmallLogM, and
   // the kernel carries the small path's registers only

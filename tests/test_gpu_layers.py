@@ -87,3 +87,34 @@ def test_batch_sorted_tiles_match_single(gpu, n, ks, precision, trials):
         top = max(abs(v) for v in want.values())
         for key, v in want.items():
             assert abs(got[key] - v) <= TOL * max(abs(v), 1e-2 * top)
+
+
+@pytest.mark.parametrize("bins", [1, 3, 125, 127, 129, 131, 253, 255, 257, 511, 513])
+def test_bin_in_time_dft_paths(gpu, orc, bins):
+    """The bin DFT's forms and their edges: direct with one (B <= 127) or two
+    (B <= 255) outputs per thread, radix-4 passes (B <= 511), Stockham."""
+    n = 1 << 14
+    rng = np.random.default_rng(bins)
+    x = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    bits = orc.num_bits(n, bins)
+    tf_o, tf = _tf(gpu, orc, n, bins)
+    ref = orc.bin_in_time(x, bins, 1e-6, bits, tf_o, 4321, version=0)
+    got = gpu.Plan(n, bins, 1e-6, bits).bin_in_time(x, tf, 4321)
+    for r in range(ref.shape[0]):
+        assert np.abs(got[r] - ref[r]).max() <= TOL * np.abs(ref[r]).max(), r
+
+
+@pytest.mark.parametrize("k", [40, 1100, 1300])
+def test_solve_many_modes_at_min_bins(gpu, orc, k):
+    """Late iterations (B = 101) with more modes than a bin-FFT workgroup
+    prefetches terms of (4 x 256): S = 1100, 1300, and few."""
+    from mpsft_amd.signals import make_signal
+    n = 1 << 18
+    x, _ = make_signal(n, k, 1e-6, seed=k)
+    s = gpu.Solver(n, gpu.solve_options(k, 1e-6))
+    s.solve(s.upload(x), 5)
+    orc.seed(5)
+    mm, _, _ = orc.demo1_run(x, k, 1e-6)
+    want, got = mm.to_dict(), s.modes_dict()
+    assert set(got) == set(want)
+    assert max(abs(got[q] - v) for q, v in want.items()) <= 1e-11
