@@ -133,6 +133,7 @@ int Batch::Prepare(const void *const *x, const uint32_t *seeds, hipStream_t s) {
   for (size_t i = 0; i < eng_.size(); ++i) {
     Engine &e = *eng_[i];
     e.rec_valid_ = false;
+    e.known_count_ = -1;
     e.defer_upload_ = &uploads_[i];
     // the first two graphs' iterations only: Run draws the rest while the
     // device works (every signal's first 32 drawn here kept the device idle
@@ -503,6 +504,7 @@ int Batch::Finish(int32_t *iters, int32_t *status, hipStream_t s) {
     } else if (r.stop_stale < opts_[i].max_stale_iter) {
       st = MPSFT_ERR_NOT_CONVERGED;
     }
+    eng_[i]->known_count_ = r.count;
     eng_[i]->FinishRecord(opts_[i], seeds_[i], st, it, r.stopped != 0);
     if (iters) iters[i] = it;
     if (status) status[i] = st;

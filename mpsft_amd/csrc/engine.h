@@ -56,6 +56,8 @@ constexpr int kSortLogBuckets = 8;  // k_bin_time's lag sort: buckets of x
 constexpr int kSortBuckets = 1 << kSortLogBuckets;
 constexpr int kSortMaxLags = 4 * kThreads;
 constexpr int kColSlices = 4;      // k_identify holds trials*rows <= 256 entries per bin
+constexpr int kProgressWords = 8;  // host-mapped words of a solve (Ctx::progress)
+constexpr size_t kModeBytes = 24;  // a found mode on its way to or from the host
 constexpr int kMaxTrials = 15;     // trials per iteration (odd)
 
 // Per-B window and bin-FFT parameters, computed on the host with the
@@ -185,7 +187,7 @@ struct Ctx {
   uint32_t *present;     // ceil(n/32) bits
   int32_t *log;          // 2 x log_cap
   int32_t *progress;     // host-mapped {iteration started, stopped, its B, and at the
-                         // stop: iterations, stale count, flags}, or null
+                         // stop: iterations, stale count, flags, found modes}, or null
   int32_t log_cap;
   int32_t cap;
   int32_t trials_cap, rows_cap, B_cap;
@@ -358,8 +360,10 @@ class Engine {
   int32_t wtab_B_ = 0;           // the window they belong to
   IdOut *d_idout_ = nullptr;     // IdentifyOnly's output pointers (device copy)
   double *d_pa_ = nullptr;       // PostAnalyze scratch: partial sums, then the stats
-  double2 *d_tmp_ = nullptr;     // cap double2 staging for mode I/O
-  int64_t *d_tmpk_ = nullptr;    // cap int64 staging for mode I/O
+  // staging for mode I/O: m coefficients (double2), then m keys (int64)
+  unsigned char *d_tmp_ = nullptr;  // cap x kModeBytes
+  std::vector<unsigned char> modes_host_;
+  int64_t known_count_ = -1;     // the map's size when the host knows it
 
   // host RNG of the transform draws (src/base.cc:32-36): std::mt19937's
   // stream, seeded lazily (a solve draws a few dozen words of the 624)

@@ -166,9 +166,9 @@ inline int32_t LagBlocks(int64_t stride) {
   const int64_t b = (stride + 4 * 256 - 1) / (4 * 256);
   return int32_t(b < 1 ? 1 : (b > 64 ? 64 : b));
 }
-hipError_t LaunchSetModes(const Ctx &c, const int64_t *keys, const double2 *coefs,
-                          int64_t m, hipStream_t s);
-hipError_t LaunchGetCoefs(const Ctx &c, double2 *out, int64_t m, hipStream_t s);
+// The map from / to a staging buffer: m coefficients (double2), then m keys.
+hipError_t LaunchSetModes(const Ctx &c, const unsigned char *in, int64_t m, hipStream_t s);
+hipError_t LaunchGetModes(const Ctx &c, unsigned char *out, int64_t m, hipStream_t s);
 // BinInFreq on a caller's rows x B matrix; limbs: rows x B x 4 integers and
 // emax two ints of scratch (the exact per-bin term sums).  emax[0] starts as
 // kNoTerms (four equal bytes, so that a byte fill sets it) and every call

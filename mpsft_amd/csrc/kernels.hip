@@ -399,7 +399,7 @@ __device__ __forceinline__ void InitBody(const Ctx &c, const InitArgs &a) {
   st->P[1].B = a.B;
   st->P[1].done = 0;
   if (c.progress)
-    for (int i = 0; i < 6; ++i)
+    for (int i = 0; i < kProgressWords; ++i)
       __hip_atomic_store(&c.progress[i], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -468,14 +468,15 @@ __device__ __forceinline__ void NextIteration(const Ctx &c, const DevFixed &fx, 
 }
 
 // The solve's result in the host-mapped progress words: iterations, stale
-// count and flags, then the iteration and the stop flag, which the host
+// count, flags and found modes, then the iteration and the stop flag, which the host
 // polls.  The release store orders the result words before the flag, so a
 // host that sees the flag reads this solve's result.
-__device__ __forceinline__ void PublishStop(const Ctx &c, int32_t it, int32_t stale,
-                                            int32_t flags) {
+__device__ __forceinline__ void PublishStop(const Ctx &c, int32_t it, int32_t stale, int32_t flags,
+                                            int32_t count) {
   __hip_atomic_store(&c.progress[3], it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&c.progress[4], stale, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&c.progress[5], flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&c.progress[6], count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&c.progress[0], it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&c.progress[1], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -516,14 +517,16 @@ __device__ void PublishLoop(const Ctx &c, int p, const IterParams &ip, const Loo
       __hip_atomic_store(&c.progress[2], ip.B, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       __hip_atomic_store(&c.progress[0], lc.it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     } else {
-      PublishStop(c, lc.it, lc.stale, st->flags);
+      PublishStop(c, lc.it, lc.stale, st->flags, st->count);
     }
   }
 }
 
-// Inserts keys/coefs into an empty map (ModeMap assignment).
+// Inserts a staging buffer's modes into an empty map (ModeMap assignment).
 __global__ void __launch_bounds__(kThreads)
-    k_set_modes(Ctx c, const int64_t *keys, const double2 *coefs, int64_t m) {
+    k_set_modes(Ctx c, const unsigned char *in, int64_t m) {
+  const double2 *coefs = reinterpret_cast<const double2 *>(in);
+  const int64_t *keys = reinterpret_cast<const int64_t *>(coefs + m);
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < m) {
     const int64_t k = keys[i];
@@ -535,9 +538,15 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 __global__ void __launch_bounds__(kThreads)
-    k_get_coefs(Ctx c, double2 *out, int64_t m) {
+    k_get_modes(Ctx c, unsigned char *out, int64_t m) {
+  double2 *coefs = reinterpret_cast<double2 *>(out);
+  int64_t *keys = reinterpret_cast<int64_t *>(coefs + m);
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < m) out[i] = c.coef[c.keys[i]];
+  if (i < m) {
+    const int64_t k = c.keys[i];
+    keys[i] = k;
+    coefs[i] = c.coef[k];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2232,7 +2241,7 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
       st->iters = lc.it;
       st->stop_stale = lc.stale;
     }
-    if (c.progress && lc.done) PublishStop(c, lc.it, lc.stale, flags);
+    if (c.progress && lc.done) PublishStop(c, lc.it, lc.stale, flags, count);
   }
   if (done) return;
   // (the launch writes P[p].done, which is not read from here on)
@@ -3445,15 +3454,14 @@ hipError_t LaunchIdentify(const Ctx &c, int parity, int32_t blocks, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t LaunchSetModes(const Ctx &c, const int64_t *keys, const double2 *coefs,
-                          int64_t m, hipStream_t s) {
-  hipLaunchKernelGGL(k_set_modes, dim3(Blocks(m)), dim3(kThreads), 0, s, c, keys, coefs, m);
+hipError_t LaunchSetModes(const Ctx &c, const unsigned char *in, int64_t m, hipStream_t s) {
+  hipLaunchKernelGGL(k_set_modes, dim3(Blocks(m)), dim3(kThreads), 0, s, c, in, m);
   return hipGetLastError();
 }
 
-hipError_t LaunchGetCoefs(const Ctx &c, double2 *out, int64_t m, hipStream_t s) {
+hipError_t LaunchGetModes(const Ctx &c, unsigned char *out, int64_t m, hipStream_t s) {
   if (m <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_get_coefs, dim3(Blocks(m)), dim3(kThreads), 0, s, c, out, m);
+  hipLaunchKernelGGL(k_get_modes, dim3(Blocks(m)), dim3(kThreads), 0, s, c, out, m);
   return hipGetLastError();
 }
 

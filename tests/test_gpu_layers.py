@@ -118,3 +118,36 @@ def test_solve_many_modes_at_min_bins(gpu, orc, k):
     want, got = mm.to_dict(), s.modes_dict()
     assert set(got) == set(want)
     assert max(abs(got[q] - v) for q, v in want.items()) <= 1e-11
+
+
+def test_mode_counts_follow_every_call(gpu):
+    """The host keeps the map's size between calls: it is right after solves,
+    Iterate, modes_set, a replay, and for a batch's signals."""
+    from mpsft_amd.signals import make_signal
+    n, k = 1 << 14, 30
+    xs = [make_signal(n, k, 1e-6, seed=s)[0] for s in (1, 2)]
+    s = gpu.Solver(n, gpu.solve_options(k, 1e-6))
+    s.set_record(True)
+    xd = [s.upload(x) for x in xs]
+    maps = []
+    for x in xd + xd:
+        s.solve(x, 4)
+        maps.append(s.modes_dict())
+    assert [len(m) for m in maps[:2]] == [len(m) for m in maps[2:]]
+    assert maps[0] == maps[2] and maps[1] == maps[3]
+    s.replay(xd[1])
+    assert set(s.modes_dict()) == set(maps[1])
+    some = dict(list(maps[0].items())[:7])
+    s.set_modes(some)
+    assert s.modes_dict() == some
+    opt = gpu.iterate_options(101, trials=1, bin_threshold=3e-7, window_threshold=0.1,
+                              sv_threshold=1e-7)
+    assert s.iterate(xd[0], opt, gpu.transform_make(n, 5, 1, 2), [3])
+    assert len(s.modes_dict()) > 7
+    s.set_modes({})
+    assert s.modes_dict() == {}
+    b = gpu.Batch([n, n], [s.opt, s.opt])
+    for seeds in ([4, 4], [5, 5], [4, 4]):
+        b.solve(xd, seeds)
+        sizes = [len(b.modes_dict(i)) for i in range(2)]
+    assert sizes == [len(maps[0]), len(maps[1])]
