@@ -3020,17 +3020,16 @@ __device__ __forceinline__ int32_t PosLagIndex(const LagGeom &L, uint32_t v) {
   return v < L.seg_end ? int32_t(v + L.sB) : PosRowIndex(L, v);
 }
 
-// Table index of offset w = -z (0 < z <= n), or -1.  Outside segment 0
-// the window is row -2^b with 2^(b-1) B < z <= 2^b B (b = ceil(log2 -lam)).
-__device__ __forceinline__ int32_t NegLagIndex(const LagGeom &L, uint32_t z) {
-  const uint32_t zp = z - 1;
+// Table index of offset w = -(zp + 1) (0 <= zp < n), or -1.  Outside segment
+// 0 the window is row -2^b with 2^(b-1) B <= zp < 2^b B (b = ceil(log2 -lam)).
+__device__ __forceinline__ int32_t NegLagIndex(const LagGeom &L, uint32_t zp) {
   int32_t d = max(31 - __clz(int32_t(zp | 1u)) - L.lb, 0);
   d -= zp < (uint32_t(L.B) << d) ? 1 : 0;  // zp < B: d = -1
-  const int32_t b = d + 1;                  // B << b <= 2 zp < 2^31 when b >= 1
-  const uint32_t off = (uint32_t(L.B) << min(b, 30)) - z;
+  const int32_t b = d + 1;                  // <= 30: zp < n <= 2^30
+  const uint32_t off = (uint32_t(L.B) << b) - 1u - zp;
   const int32_t row =
       ((b < L.bits) & (off < L.fB)) ? L.neg0 + b * int32_t(L.fB) + int32_t(off) : -1;
-  return z <= L.sB ? int32_t(L.sB - z) : row;
+  return zp < L.sB ? int32_t(L.sB - 1u - zp) : row;
 }
 
 // The table is E / B slots of B residues: slot sigma holds lag lam (offsets
@@ -3045,6 +3044,42 @@ __device__ __forceinline__ int32_t SlotLag(const LagGeom &L, int32_t sigma) {
   return r < rows ? (1 << (L.K + r)) + k : k - (1 << (L.K + r - rows));
 }
 
+// One (iteration, trial) of AdjGatherBody32: the lookups of a thread's
+// kGatherJ samples, whose offsets are v0 + q vstep (mod n).  kWrap: offsets
+// v < L.top stand for w = v + n too.
+template <bool kWrap>
+__device__ __forceinline__ void AdjGatherTrial(const LagGeom &L, const double2 *tab, uint32_t n,
+                                               uint32_t v0, uint32_t vstep,
+                                               const bool (&in)[kGatherJ],
+                                               double2 (&acc)[kGatherJ]) {
+  constexpr int R = kWrap ? 3 : 2;
+  const uint32_t m32 = n - 1;
+  // every lookup of the kGatherJ samples is issued before any is added; only
+  // lanes with a window load (a miss adds +0, which leaves a sum that
+  // started at +0 unchanged)
+  int32_t idx[kGatherJ][R];
+  double2 val[kGatherJ][R];
+#pragma unroll
+  for (int q = 0; q < kGatherJ; ++q) {
+    const uint32_t v = (v0 + uint32_t(q) * vstep) & m32;
+    const bool wrap = kWrap && int32_t(v) < L.top;
+    const uint32_t w = wrap ? v + n : v;
+    const int32_t p = PosLagIndex(L, w);
+    idx[q][0] = in[q] ? NegLagIndex(L, m32 - v) : -1;
+    idx[q][1] = !in[q] ? -1 : (wrap ? int32_t(v + L.sB) : p);
+    if (kWrap) idx[q][R - 1] = (in[q] & wrap) ? p : -1;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      val[q][r] = make_double2(0.0, 0.0);
+      if (idx[q][r] >= 0) val[q][r] = LoadX<false>(tab + idx[q][r]);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kGatherJ; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[q] = Add(acc[q], val[q][r]);
+}
+
 // AdjGatherBody for n = 2^k <= 2^30 with the lag tables of k_adj_lags: per
 // sample and recorded (iteration, trial), the offset v = u - base of its
 // permuted index u (the low bits of 32-bit products) is looked up as
@@ -3053,57 +3088,45 @@ __device__ __forceinline__ int32_t SlotLag(const LagGeom &L, int32_t sigma) {
 // lies in [-n, n + f B) since 2^(bits-1) B <= n (bits = 1 + floor(log2(n /
 // B))), in increasing order.  top <= f B <= (s0 + f) B, so for v < top the
 // offset w = v is in segment 0 and only w = v + n needs the general lookup.
+// Most iterations have top <= 0 and leave that lookup out.
+// Bound by the integer instructions of the lookups (most offsets miss every
+// window): per thread and trial one product, the further samples' offsets by
+// adding gsize a_inv, and the iteration's parameters in scalar registers.
+// 32 signals of n = 2^20 (100 modes): 611 -> 500 us.
 template <typename Tout>
 __device__ __forceinline__ void AdjGatherBody32(const Ctx &c, const AdjSig &g, const AdjStep *steps,
                                                 int32_t count, int32_t si, Tout *out, int64_t tid,
                                                 int64_t gsize) {
   const uint32_t n = uint32_t(c.n);
-  const uint32_t m32 = n - 1;
   for (int64_t j0 = tid; j0 < int64_t(n); j0 += gsize * kGatherJ) {
     double2 acc[kGatherJ];
+    bool in[kGatherJ];
 #pragma unroll
-    for (int q = 0; q < kGatherJ; ++q) acc[q] = make_double2(0.0, 0.0);
+    for (int q = 0; q < kGatherJ; ++q) {
+      acc[q] = make_double2(0.0, 0.0);
+      in[q] = j0 + q * gsize < int64_t(n);
+    }
     for (int32_t s = 0; s < g.iters; ++s) {
       const AdjStep &st = steps[int64_t(s) * count + si];
-      if (!st.active) continue;
-      const IterParams &ip = st.ip;
+      if (!LoadUniform(&st.active)) continue;
+      const IterParams ip = LoadUniform(&st.ip);
       const LagGeom L = MakeLagGeom(ip, n);
       const uint32_t a_inv = uint32_t(ip.tf.a_inv), cc = uint32_t(ip.tf.c);
-      for (int32_t t = 0; t < st.trials; ++t) {
-        const uint32_t base = uint32_t(ip.q[t] - ip.p2) & m32;
-        const double2 *tab = g.lags + (int64_t(st.it) * c.trials_cap + t) * g.lags_stride;
-        // every lookup of the kGatherJ samples is issued before any is
-        // added; only lanes with a window load (a miss adds +0, which
-        // leaves a sum that started at +0 unchanged)
-        int32_t idx[kGatherJ][3];
-        double2 val[kGatherJ][3];
-#pragma unroll
-        for (int q = 0; q < kGatherJ; ++q) {
-          const int64_t j = j0 + q * gsize;
-          const uint32_t u = (a_inv * ((uint32_t(j) - cc) & m32)) & m32;
-          const uint32_t v = (u - base) & m32;
-          const bool in = j < int64_t(n), wrap = int32_t(v) < L.top;
-          const uint32_t w = wrap ? v + n : v;
-          const int32_t p = w < L.seg_end ? int32_t(w + L.sB) : PosRowIndex(L, w);
-          idx[q][0] = in ? NegLagIndex(L, n - v) : -1;
-          idx[q][1] = !in ? -1 : (wrap ? int32_t(v + L.sB) : p);
-          idx[q][2] = (in & wrap) ? p : -1;
-#pragma unroll
-          for (int r = 0; r < 3; ++r) {
-            val[q][r] = make_double2(0.0, 0.0);
-            if (idx[q][r] >= 0) val[q][r] = LoadX<false>(tab + idx[q][r]);
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < kGatherJ; ++q)
-#pragma unroll
-          for (int r = 0; r < 3; ++r) acc[q] = Add(acc[q], val[q][r]);
+      const uint32_t u0 = a_inv * (uint32_t(j0) - cc), vstep = a_inv * uint32_t(gsize);
+      const int32_t trials = LoadUniform(&st.trials), it = LoadUniform(&st.it);
+      for (int32_t t = 0; t < trials; ++t) {
+        const uint32_t v0 = u0 - uint32_t(LoadUniform(&st.ip.q[t]) - ip.p2);
+        const double2 *tab = g.lags + (int64_t(it) * c.trials_cap + t) * g.lags_stride;
+        if (L.top > 0)
+          AdjGatherTrial<true>(L, tab, n, v0, vstep, in, acc);
+        else
+          AdjGatherTrial<false>(L, tab, n, v0, vstep, in, acc);
       }
     }
 #pragma unroll
     for (int q = 0; q < kGatherJ; ++q) {
       const int64_t j = j0 + q * gsize;
-      if (j < int64_t(n)) {
+      if (in[q]) {
         out[j].x = acc[q].x;
         out[j].y = acc[q].y;
       }

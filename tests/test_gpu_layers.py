@@ -151,3 +151,30 @@ def test_mode_counts_follow_every_call(gpu):
         b.solve(xd, seeds)
         sizes = [len(b.modes_dict(i)) for i in range(2)]
     assert sizes == [len(maps[0]), len(maps[1])]
+
+
+@pytest.mark.parametrize("n,k,min_bins,precision", [
+    (1 << 16, 50, 101, 0),  # 2^(bits-1) B + f B below n: offsets have one positive lag
+    (1 << 16, 50, 127, 0),  # above n: offsets below f B have two
+    (1 << 16, 50, 129, 1),
+    (1 << 9, 3, 7, 0),      # fewer samples than a workgroup's threads x 4
+])
+def test_adjoint_gather_ranges(gpu, n, k, min_bins, precision):
+    """<F d, g> = <d, F^H g> on both forms of the adjoint's table gather."""
+    from mpsft_amd.signals import make_signal
+    x, _ = make_signal(n, k, 1e-6, seed=3)
+    s = gpu.Solver(n, gpu.solve_options(k, 1e-5, min_bins=min_bins),
+                   gpu.MPSFT_MIXED if precision else gpu.MPSFT_FP64)
+    s.set_record(True)
+    s.solve(s.upload(x.astype(np.complex64) if precision else x), 5)
+    keys, _ = s.modes()
+    rng = np.random.default_rng(13)
+    d = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    s.replay(gpu.DeviceArray.from_numpy(d), precision=gpu.MPSFT_FP64)
+    fd = s.modes_dict()
+    fd = np.array([fd[int(q)] for q in keys])
+    g = rng.standard_normal(keys.size) + 1j * rng.standard_normal(keys.size)
+    adj = s.adjoint(keys, g)
+    assert keys.size >= k // 2
+    tol = TOL * (np.linalg.norm(g) * np.linalg.norm(fd) + np.linalg.norm(adj) * np.linalg.norm(d))
+    assert abs(np.vdot(g, fd) - np.vdot(adj, d)) <= tol
