@@ -1146,7 +1146,12 @@ struct TermGrid {
   double scale, inv;  // 2^(94-E), 2^(E-94)
   bool any;           // some term is nonzero
 };
-constexpr int kLimbs = 4;  // per bin: re h, re l, im h, im l
+// Per bin: re h, re l, im h, im l.  In LDS limb l of bin b sits at l B + b, so
+// that the 64 atomics of a wavefront spread over every bank; at 4 b + l they
+// meet on an eighth of them (64 signals of n = 2^22 per batched solve:
+// small-path launches 24.3 -> 22.7 us, large-path 79.6 -> 76.7, the solve
+// 7078 -> 7025).
+constexpr int kLimbs = 4;
 
 // The workgroup's largest term component (each thread its v) -> the grid.
 // Every thread calls it.  The lanes compare exponents, one word per shuffle.
@@ -1169,25 +1174,28 @@ __device__ __forceinline__ TermGrid MakeTermGrid(double v) {
 
 __device__ __forceinline__ double MaxComp(double2 v) { return fmax(fabs(v.x), fabs(v.y)); }
 
-__device__ __forceinline__ void LimbAdd(unsigned long long *acc, double2 v, const TermGrid &g) {
+__device__ __forceinline__ void LimbAdd(unsigned long long *acc, int stride, double2 v,
+                                        const TermGrid &g) {
   const double comp[2] = {v.x, v.y};
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const double x = comp[j] * g.scale;
     const double h = trunc(x * 0x1p-47);
     const double l = rint(x - h * 0x1p47);
-    atomicAdd(&acc[2 * j], static_cast<unsigned long long>(static_cast<long long>(h)));
-    atomicAdd(&acc[2 * j + 1], static_cast<unsigned long long>(static_cast<long long>(l)));
+    atomicAdd(&acc[2 * j * stride], static_cast<unsigned long long>(static_cast<long long>(h)));
+    atomicAdd(&acc[(2 * j + 1) * stride],
+              static_cast<unsigned long long>(static_cast<long long>(l)));
   }
 }
 
 // The bin's accumulated terms as a double2 (one rounding per component).
-__device__ __forceinline__ double2 LimbValue(const unsigned long long *acc, const TermGrid &g) {
+__device__ __forceinline__ double2 LimbValue(const unsigned long long *acc, int stride,
+                                             const TermGrid &g) {
   double out[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    long long h = static_cast<long long>(acc[2 * j]);
-    long long l = static_cast<long long>(acc[2 * j + 1]);
+    long long h = static_cast<long long>(acc[2 * j * stride]);
+    long long l = static_cast<long long>(acc[(2 * j + 1) * stride]);
     const long long carry = l >> 47;  // floor(l / 2^47): 0 <= l < 2^47 after it
     l -= carry * (1ll << 47);
     h += carry;
@@ -1233,7 +1241,7 @@ __device__ __forceinline__ void StoreBins(double2 *A, int32_t B, const double2 (
 #pragma unroll
   for (int r = 0; r < N; ++r) {
     const int k = threadIdx.x + r * kFftThreads;
-    if (k < B) A[k] = g.any ? Sub(xo[r], LimbValue(limbs + kLimbs * k, g)) : xo[r];
+    if (k < B) A[k] = g.any ? Sub(xo[r], LimbValue(limbs + k, B, g)) : xo[r];
   }
 }
 
@@ -1550,11 +1558,11 @@ __device__ __forceinline__ void DirectRow(int32_t B, const DirectIn &in, double2
   if (g.any) {
 #pragma unroll
     for (int r = 0; r < N; ++r)
-      if (tid + r * T < cnt) LimbAdd(l->limbs + kLimbs * bin[r], val[r], g);
+      if (tid + r * T < cnt) LimbAdd(l->limbs + bin[r], B, val[r], g);
     for (int i = tid + N * T; i < cnt; i += T) {
       int32_t b;
       const double2 v = term(i, &b);
-      LimbAdd(l->limbs + kLimbs * b, v, g);
+      LimbAdd(l->limbs + b, B, v, g);
     }
   }
   DirectOut out;
@@ -1563,7 +1571,7 @@ __device__ __forceinline__ void DirectRow(int32_t B, const DirectIn &in, double2
 #pragma unroll
   for (int i = 0; i < kDirectPer; ++i)
     if (out.k[i] >= 0)
-      A[out.k[i]] = g.any ? Sub(out.x[i], LimbValue(l->limbs + kLimbs * out.k[i], g)) : out.x[i];
+      A[out.k[i]] = g.any ? Sub(out.x[i], LimbValue(l->limbs + out.k[i], B, g)) : out.x[i];
 }
 
 template <int kPaths>
@@ -1640,8 +1648,8 @@ __device__ __forceinline__ void BinFftBody(const Ctx &c, int p, int blk, double2
   if (g.any) {
 #pragma unroll
     for (int r = 0; r < kPerTerm; ++r)
-      if (tid + r * T < cnt) LimbAdd(limbs + kLimbs * tbin[r], tval[r], g);
-    for (int i = tid + kPerTerm * T; i < cnt; i += T) LimbAdd(limbs + kLimbs * tb[i], tv[i], g);
+      if (tid + r * T < cnt) LimbAdd(limbs + tbin[r], B, tval[r], g);
+    for (int i = tid + kPerTerm * T; i < cnt; i += T) LimbAdd(limbs + tb[i], B, tv[i], g);
   }
   __syncthreads();
   StoreBins(A, B, xo, limbs, g);
@@ -1839,7 +1847,7 @@ __global__ void __launch_bounds__(kThreads) k_big_out(Ctx c, int p) {
         const int bin = tb[i];
         const int col = (bin & (G.N2 - 1)) - n2_0;
         const int li = (col << G.logN1) + (bin >> G.logN2) - h * kHalf;
-        if (col >= 0 && col < C && li >= 0 && li < kHalf) LimbAdd(limbs + kLimbs * li, tv[i], tg);
+        if (col >= 0 && col < C && li >= 0 && li < kHalf) LimbAdd(limbs + li, kHalf, tv[i], tg);
       }
       __syncthreads();
     }
@@ -1850,7 +1858,7 @@ __global__ void __launch_bounds__(kThreads) k_big_out(Ctx c, int p) {
       const int m = (n1 << G.logN2) + n2_0 + col;
       const int li = (col << G.logN1) + n1 - h * kHalf;
       if (m < B && li >= 0 && li < kHalf)
-        A[m] = tg.any ? Sub(xo[r], LimbValue(limbs + kLimbs * li, tg)) : xo[r];
+        A[m] = tg.any ? Sub(xo[r], LimbValue(limbs + li, kHalf, tg)) : xo[r];
     }
     if (tg.any) __syncthreads();  // the limbs are read before the next half clears them
   }
@@ -2358,12 +2366,12 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
   if (g.any) {
 #pragma unroll
     for (int r = 0; r < kPerTerm; ++r)
-      if (tid + r * T < cnt) LimbAdd(limbs + kLimbs * tbin[r], vr[r], g);
+      if (tid + r * T < cnt) LimbAdd(limbs + tbin[r], B, vr[r], g);
     for (int i = tid + kPerTerm * T; i < cnt; i += T) {
       int32_t bin;
       const int64_t k0 = c.keys[i];
       const double2 v = term(i, k0, c.coef[k0], &bin);
-      LimbAdd(limbs + kLimbs * bin, v, g);
+      LimbAdd(limbs + bin, B, v, g);
     }
   }
   __syncthreads();
@@ -2450,9 +2458,9 @@ __global__ void __launch_bounds__(kThreads)
     const double2 base = Cmul(d.cw, CisFrac(ModN(q * d.k1 + tf.c * d.k0, n, mask), n));
     const double2 t = CisFrac(ModN((int64_t(bp.B) << bit) * d.k1, n, mask), n);
     unsigned long long *acc = limbs + kLimbs * (int64_t(2 * bit + 1) * bp.B + d.bin);
-    if (bit == 0) LimbAdd(limbs + kLimbs * int64_t(d.bin), base, g);
-    LimbAdd(acc, Cmul(base, t), g);
-    LimbAdd(acc + kLimbs * int64_t(bp.B), Cmul(base, Conj(t)), g);
+    if (bit == 0) LimbAdd(limbs + kLimbs * int64_t(d.bin), 1, base, g);
+    LimbAdd(acc, 1, Cmul(base, t), g);
+    LimbAdd(acc + kLimbs * int64_t(bp.B), 1, Cmul(base, Conj(t)), g);
   }
 }
 
@@ -2465,7 +2473,7 @@ __global__ void __launch_bounds__(kThreads)
   if (i == 0) emax[0] = kNoTerms;
   if (!g.any) return;
   for (int64_t j = i; j < count; j += int64_t(gridDim.x) * blockDim.x)
-    out[j] = Sub(out[j], LimbValue(limbs + kLimbs * j, g));
+    out[j] = Sub(out[j], LimbValue(limbs + kLimbs * j, 1, g));
 }
 
 __global__ void __launch_bounds__(kThreads)
