@@ -1543,12 +1543,12 @@ __device__ __forceinline__ void DirectDft(int32_t B, double2 rp, const DirectLds
 }
 
 // DFT, row phase and BinInFreq of one row.  val, bin: this thread's first N
-// terms (modes threadIdx.x + r kFftThreads < cnt); term(i, &bin) forms any
-// later one; mx: the largest component of all the thread's terms.
-template <int N, typename Term>
+// terms (modes threadIdx.x + r kFftThreads < cnt); rest(use) calls use(bin,
+// term) for its later ones; mx: the largest component of all its terms.
+template <int N, typename Rest>
 __device__ __forceinline__ void DirectRow(int32_t B, const DirectIn &in, double2 rp, double2 *lds,
                                           const double2 (&val)[N], const int (&bin)[N],
-                                          int32_t cnt, double mx, Term term, double2 *A) {
+                                          int32_t cnt, double mx, Rest rest, double2 *A) {
   constexpr int T = kFftThreads;
   DirectLds *l = reinterpret_cast<DirectLds *>(lds);
   const int tid = threadIdx.x;
@@ -1559,11 +1559,7 @@ __device__ __forceinline__ void DirectRow(int32_t B, const DirectIn &in, double2
 #pragma unroll
     for (int r = 0; r < N; ++r)
       if (tid + r * T < cnt) LimbAdd(l->limbs + bin[r], B, val[r], g);
-    for (int i = tid + N * T; i < cnt; i += T) {
-      int32_t b;
-      const double2 v = term(i, &b);
-      LimbAdd(l->limbs + b, B, v, g);
-    }
+    rest([&](int b, const double2 &v) { LimbAdd(l->limbs + b, B, v, g); });
   }
   DirectOut out;
   DirectDft(B, rp, l, &out);
@@ -1617,9 +1613,8 @@ __device__ __forceinline__ void BinFftBody(const Ctx &c, int p, int blk, double2
   double2 *A = c.A + (int64_t(trial) * c.rows_cap + row) * c.B_cap;
   if (direct) {
     DirectRow(B, in, rp, lds, tval, tbin, cnt, mx,
-              [&](int i, int32_t *bin) {
-                *bin = tb[i];
-                return tv[i];
+              [&](auto use) {
+                for (int i = tid + kPerTerm * T; i < cnt; i += T) use(tb[i], tv[i]);
               },
               A);
     return;
@@ -2306,14 +2301,41 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
 #pragma unroll
   for (int r = 0; r < kPerTerm; ++r) cfv[r] = kk[r] >= 0 ? c.coef[kk[r]] : make_double2(0.0, 0.0);
   // The terms of the first modes are formed once, in registers, and the rest
-  // (more than kPerTerm x T modes) are formed again for the second pass.
-  auto term = [&](int i, int64_t k0, const double2 &cf, int32_t *bin) {
-    if (i < cnt_pre) {
-      *bin = tb[i];
-      return Cmul(cf, tv[i]);
+  // (more than kPerTerm x T modes) by rest(use) in each of the two passes:
+  // those with a factor kPerTerm at a time, their loads in flight together
+  // (a key, then its coefficient at a random place; one by one a launch with
+  // 4000 modes takes 15.7 us, so 12.5, and the solve 1417 -> 1361), then the few
+  // modes found since.
+  auto rest = [&](auto use) {
+    const int32_t with = min(cnt_pre, cnt);
+    for (int i0 = tid + kPerTerm * T; i0 < with; i0 += kPerTerm * T) {
+      double2 f[kPerTerm], cf[kPerTerm];
+      int b[kPerTerm];
+      int64_t k[kPerTerm];
+#pragma unroll
+      for (int r = 0; r < kPerTerm; ++r) {
+        const int i = i0 + r * T;
+        k[r] = -1;
+        if (i < with) {
+          k[r] = c.keys[i];
+          f[r] = tv[i];
+          b[r] = tb[i];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < kPerTerm; ++r)
+        if (k[r] >= 0) cf[r] = c.coef[k[r]];
+#pragma unroll
+      for (int r = 0; r < kPerTerm; ++r)
+        if (k[r] >= 0) use(b[r], Cmul(cf[r], f[r]));
     }
-    const int64_t k1 = ModN(ip.tf.a * k0 + ip.tf.b, n, mask);
-    return Cmul(cf, RowFactor(c, ip, q, row, k0, k1, bin));
+    for (int i = max(with, kPerTerm * T) + tid; i < cnt; i += T) {
+      const int64_t k0 = c.keys[i];
+      const int64_t k1 = ModN(ip.tf.a * k0 + ip.tf.b, n, mask);
+      int32_t bin;
+      const double2 f = RowFactor(c, ip, q, row, k0, k1, &bin);
+      use(bin, Cmul(c.coef[k0], f));
+    }
   };
   double2 vr[kPerTerm];
   double mx = 0.0;
@@ -2331,19 +2353,10 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
       mx = fmax(mx, MaxComp(vr[r]));
     }
   }
-  for (int i = tid + kPerTerm * T; i < cnt; i += T) {
-    int32_t bin;
-    const int64_t k0 = c.keys[i];
-    mx = fmax(mx, MaxComp(term(i, k0, c.coef[k0], &bin)));
-  }
+  rest([&](int, const double2 &v) { mx = fmax(mx, MaxComp(v)); });
   double2 *A = c.A + (int64_t(trial) * c.rows_cap + row) * c.B_cap;
   if (direct) {
-    DirectRow(B, in, rp, lds, vr, tbin, cnt, mx,
-              [&](int i, int32_t *bin) {
-                const int64_t k0 = c.keys[i];
-                return term(i, k0, c.coef[k0], bin);
-              },
-              A);
+    DirectRow(B, in, rp, lds, vr, tbin, cnt, mx, rest, A);
     return;
   }
   double2 *a = lds;
@@ -2367,12 +2380,7 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
 #pragma unroll
     for (int r = 0; r < kPerTerm; ++r)
       if (tid + r * T < cnt) LimbAdd(limbs + tbin[r], B, vr[r], g);
-    for (int i = tid + kPerTerm * T; i < cnt; i += T) {
-      int32_t bin;
-      const int64_t k0 = c.keys[i];
-      const double2 v = term(i, k0, c.coef[k0], &bin);
-      LimbAdd(limbs + bin, B, v, g);
-    }
+    rest([&](int b, const double2 &v) { LimbAdd(limbs + b, B, v, g); });
   }
   __syncthreads();
   StoreBins(A, B, xo, limbs, g);
