@@ -141,13 +141,10 @@ int mpsft_plan_create(int64_t n, int32_t bins, double delta, int32_t bits, int p
   const size_t limbs = size_t(1 + 2 * bits) * bins * 4;
   if (hipMalloc(reinterpret_cast<void **>(&p->d_limbs), limbs * sizeof(unsigned long long)) !=
           hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&p->d_emax), 2 * sizeof(int32_t)) != hipSuccess) {
+      hipMalloc(reinterpret_cast<void **>(&p->d_emax), (mpsft::kFreqSlots + 1) * sizeof(int32_t)) !=
+          hipSuccess) {
     mpsft_plan_destroy(p);
     return MPSFT_ERR_NOMEM;
-  }
-  if (hipMemset(p->d_emax, mpsft::kNoTermsByte, 2 * sizeof(int32_t)) != hipSuccess) {
-    mpsft_plan_destroy(p);
-    return MPSFT_ERR_HIP;
   }
   *plan = p;
   return MPSFT_OK;

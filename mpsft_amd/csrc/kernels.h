@@ -170,11 +170,8 @@ inline int32_t LagBlocks(int64_t stride) {
 hipError_t LaunchSetModes(const Ctx &c, const unsigned char *in, int64_t m, hipStream_t s);
 hipError_t LaunchGetModes(const Ctx &c, unsigned char *out, int64_t m, hipStream_t s);
 // BinInFreq on a caller's rows x B matrix; limbs: rows x B x 4 integers and
-// emax two ints of scratch (the exact per-bin term sums).  emax[0] starts as
-// kNoTerms (four equal bytes, so that a byte fill sets it) and every call
-// leaves it so.
-constexpr int kNoTermsByte = 0x80;
-constexpr int32_t kNoTerms = int32_t(0x80808080u);
+// emax kFreqSlots + 1 ints of scratch (the exact per-bin term sums).
+constexpr int32_t kFreqSlots = 512;
 hipError_t LaunchBinInFreqDirect(int64_t n, int64_t mask, const BParams &bp,
                                  const DevTf &tf, int64_t q, const int64_t *k0,
                                  const double2 *coef, int64_t m, double2 *out,

@@ -2394,9 +2394,10 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
 // BinInFreqV1 (src/binner.cc:565-591) on a caller-owned bin matrix (rows x
 // B, row stride B), with each bin's terms summed exactly as in the solve
 // (TermGrid) so the result does not depend on the order of the modes or of
-// the threads: a pass for the grid exponent (by atomicMax), a pass adding
-// the limbs into limbs[(row B + bin) kLimbs ...], and one subtracting each
-// bin's sum.
+// the threads: a pass for the grid exponent, a pass adding the limbs into
+// limbs[(row B + bin) kLimbs ...], and one subtracting each bin's sum.  Each
+// pass writes the scratch that the next one reads, so a call depends on
+// nothing that was in it before.
 //
 // Bound by latency: a term costs two erf and two sincospi, 2 x 4 integer
 // atomics follow, and there are few modes.  So a thread takes one (mode,
@@ -2423,9 +2424,19 @@ __device__ __forceinline__ DirectMode DirectBase(int64_t n, int64_t mask, const 
   return d;
 }
 
-// limbs[0..count) = 0 (a kernel rather than a memset), and emax[0] = the
-// exponent of the largest |coef| wf (emax[0] is kNoTerms before: from the
-// plan's creation or the previous call's last pass).
+// The largest of every thread's exponent, in every thread (kThreads of them).
+__device__ __forceinline__ int32_t BlockMax(int32_t e) {
+  __shared__ int32_t wmax[kThreads / 64];
+  for (int off = 1; off < 64; off <<= 1) e = max(e, __shfl(e, int(threadIdx.x ^ off) & 63));
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = e;
+  __syncthreads();
+  for (int w = 0; w < kThreads / 64; ++w) e = max(e, wmax[w]);
+  return e;
+}
+
+// limbs[0..count) = 0 (a kernel rather than a memset), and emax[blockIdx.x] =
+// the exponent of the workgroup's largest |coef| wf (kNoTerms if all are 0).
+constexpr int32_t kNoTerms = -(1 << 30);
 __global__ void __launch_bounds__(kThreads)
     k_freq_direct_max(int64_t n, int64_t mask, BParams bp, DevTf tf, const int64_t *k0s,
                       const double2 *coefs, int64_t m, int32_t *emax, unsigned long long *limbs,
@@ -2438,8 +2449,8 @@ __global__ void __launch_bounds__(kThreads)
     const DirectMode d = DirectBase(n, mask, bp, tf, k0s[j], coefs[j]);
     mx = fmax(mx, hypot(d.cw.x, d.cw.y));
   }
-  for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
-  if ((threadIdx.x & 63) == 0 && mx > 0.0) atomicMax(emax, ilogb(mx) + 1);
+  const int32_t e = BlockMax(mx > 0.0 ? ilogb(mx) + 1 : kNoTerms);
+  if (threadIdx.x == 0) emax[blockIdx.x] = e;
 }
 
 // The grid of exponent e (every term component below 2^e); e = kNoTerms
@@ -2452,14 +2463,17 @@ __device__ __forceinline__ TermGrid TermGridOf(int32_t e) {
   return g;
 }
 
-// One (mode, bit) per thread.  emax[1] = emax[0] for the last pass.
+// One (mode, bit) per thread.  emax: the first pass's `slots` exponents;
+// their largest goes to emax[kFreqSlots], for the last pass.
 __global__ void __launch_bounds__(kThreads)
     k_freq_direct_add(int64_t n, int64_t mask, BParams bp, DevTf tf, int64_t q,
                       const int64_t *k0s, const double2 *coefs, int64_t m, int32_t *emax,
-                      unsigned long long *limbs) {
+                      int32_t slots, unsigned long long *limbs) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int32_t e = emax[0];
-  if (i == 0) emax[1] = e;
+  int32_t e = kNoTerms;
+  for (int32_t k = threadIdx.x; k < slots; k += kThreads) e = max(e, emax[k]);
+  e = BlockMax(e);
+  if (i == 0) emax[kFreqSlots] = e;
   const TermGrid g = TermGridOf(e);
   const int64_t work = m * bp.bits;
   if (!g.any) return;
@@ -2477,13 +2491,12 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-// out -= the bins' sums; emax[0] is left ready for the next call.
+// out -= the bins' sums.
 __global__ void __launch_bounds__(kThreads)
-    k_freq_direct_sub(const unsigned long long *limbs, int32_t *emax, int64_t count,
+    k_freq_direct_sub(const unsigned long long *limbs, const int32_t *emax, int64_t count,
                       double2 *out) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const TermGrid g = TermGridOf(emax[1]);
-  if (i == 0) emax[0] = kNoTerms;
+  const TermGrid g = TermGridOf(emax[kFreqSlots]);
   if (!g.any) return;
   for (int64_t j = i; j < count; j += int64_t(gridDim.x) * blockDim.x)
     out[j] = Sub(out[j], LimbValue(limbs + kLimbs * j, 1, g));
@@ -3531,10 +3544,11 @@ hipError_t LaunchBinInFreqDirect(int64_t n, int64_t mask, const BParams &bp,
                                  unsigned long long *limbs, int32_t *emax, hipStream_t s) {
   if (m <= 0) return hipSuccess;
   const int64_t bins = int64_t(1 + 2 * bp.bits) * bp.B;
-  hipLaunchKernelGGL(k_freq_direct_max, dim3(Blocks(std::max(kLimbs * bins, m))), dim3(kThreads), 0,
-                     s, n, mask, bp, tf, k0, coef, m, emax, limbs, kLimbs * bins);
+  const int32_t slots = std::min(Blocks(std::max(kLimbs * bins, m)), kFreqSlots);
+  hipLaunchKernelGGL(k_freq_direct_max, dim3(slots), dim3(kThreads), 0, s, n, mask, bp, tf, k0, coef,
+                     m, emax, limbs, kLimbs * bins);
   hipLaunchKernelGGL(k_freq_direct_add, dim3(Blocks(m * bp.bits)), dim3(kThreads), 0, s, n, mask, bp,
-                     tf, q, k0, coef, m, emax, limbs);
+                     tf, q, k0, coef, m, emax, slots, limbs);
   hipLaunchKernelGGL(k_freq_direct_sub, dim3(Blocks(bins)), dim3(kThreads), 0, s, limbs, emax, bins,
                      out);
   return hipGetLastError();

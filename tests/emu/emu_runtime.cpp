@@ -303,6 +303,26 @@ bool Tracked(const void *p) {
   return a < it->first + it->second;
 }
 
+// EMU_GARBAGE: the byte that new device memory is filled with (0xa5).
+// EMU_LATE_FILL=1: hipMemset returns before its fill, which then waits for
+// the host to wait for the device, as HIP allows for device memory; work on
+// a non-blocking stream runs ahead of it.
+int EnvByte(const char *name, int def) {
+  const char *e = std::getenv(name);
+  return e ? int(std::strtol(e, nullptr, 0)) : def;
+}
+std::mutex g_fill_mu;
+std::vector<std::function<void()>> g_late_fills;
+
+void RunLateFills() {
+  std::vector<std::function<void()>> f;
+  {
+    std::lock_guard<std::mutex> lk(g_fill_mu);
+    f.swap(g_late_fills);
+  }
+  for (auto &fill : f) fill();
+}
+
 Device &Dev() {
   // Never destroyed: the worker thread may outlive static destructors.
   static Device *d = [] {
@@ -339,12 +359,13 @@ hipError_t hipGetSymbolAddress(void **p, const void *symbol) {
 hipError_t hipMalloc(void **p, size_t bytes) {
   *p = nullptr;
   if (posix_memalign(p, 256, bytes ? bytes : 1) != 0) return hipErrorOutOfMemory;
-  std::memset(*p, 0xa5, bytes);  // device memory starts as garbage
+  std::memset(*p, EnvByte("EMU_GARBAGE", 0xa5), bytes);  // device memory starts as garbage
   Track(*p, bytes ? bytes : 1);
   return hipSuccess;
 }
 hipError_t hipFree(void *p) {
   Dev().Wait();
+  RunLateFills();
   if (p) Untrack(p);
   std::free(p);
   return hipSuccess;
@@ -357,6 +378,7 @@ hipError_t hipHostGetDevicePointer(void **dev, void *host, unsigned) {
 }
 hipError_t hipMemcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind) {
   Dev().Wait();
+  RunLateFills();
   if (bytes) std::memcpy(dst, src, bytes);
   return hipSuccess;
 }
@@ -379,7 +401,13 @@ hipError_t hipMemcpy2D(void *dst, size_t dpitch, const void *src, size_t spitch,
 }
 hipError_t hipMemset(void *dst, int value, size_t bytes) {
   Dev().Wait();
-  if (bytes) std::memset(dst, value, bytes);
+  if (!bytes) return hipSuccess;
+  if (EnvByte("EMU_LATE_FILL", 0)) {
+    std::lock_guard<std::mutex> lk(g_fill_mu);
+    g_late_fills.push_back([=] { std::memset(dst, value, bytes); });
+    return hipSuccess;
+  }
+  std::memset(dst, value, bytes);
   return hipSuccess;
 }
 hipError_t hipMemsetAsync(void *dst, int value, size_t bytes, hipStream_t) {
@@ -389,6 +417,7 @@ hipError_t hipMemsetAsync(void *dst, int value, size_t bytes, hipStream_t) {
 }
 hipError_t hipDeviceSynchronize() {
   Dev().Wait();
+  RunLateFills();
   return hipSuccess;
 }
 hipError_t hipStreamCreate(hipStream_t *s) {
@@ -401,8 +430,9 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   delete s;
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) {
+hipError_t hipStreamSynchronize(hipStream_t s) {
   Dev().Wait();
+  if (!s) RunLateFills();
   return hipSuccess;
 }
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {

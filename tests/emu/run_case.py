@@ -111,6 +111,25 @@ def plan_freq(n, bins, bits, m, seed):
                 identical=bool(np.array_equal(got.view(np.float64), got2.view(np.float64))))
 
 
+def plan_freq_first(n, bins, bits, m, seed):
+    """BinInFreq as a fresh plan's first call, on a non-blocking stream."""
+    rng = np.random.default_rng(seed)
+    keys = rng.choice(n, m, replace=False).astype(np.int64)
+    coefs = rng.standard_normal(m) + 1j * rng.standard_normal(m)
+    base = rng.standard_normal((1 + 2 * bits, bins)) + 1j * rng.standard_normal((1 + 2 * bits, bins))
+    orc.seed(seed)
+    tf = orc.transform_draw(n)
+    ref = orc.bin_in_freq(keys, coefs, n, bins, 1e-6, bits, tf, 5, base.copy(), version=0)
+    kd, cd, od = (gpu.DeviceArray.from_numpy(v) for v in (keys, coefs, base))
+    stream = C.c_void_p()
+    gpu.lib().mpsft_stream_create(C.byref(stream))
+    p = gpu.Plan(n, bins, 1e-6, bits)
+    p.bin_in_freq_dev(kd, cd, m, gpu.transform_make(n, *map(int, tf[:3])), 5, od, stream)
+    gpu.lib().mpsft_stream_synchronize(stream)
+    got = od.to_numpy(np.complex128, base.shape)
+    return dict(abs_err=float(np.abs(got - ref).max()), scale=float(np.abs(ref).max()))
+
+
 def batch(ns, ks, sigma, seeds, precision=0, autotune=False):
     xs = [signal(n, k, sigma, sd) for n, k, sd in zip(ns, ks, seeds)]
     xg = [x.astype(np.complex64) if precision else x for x in xs]
@@ -276,5 +295,6 @@ if __name__ == "__main__":
     os.environ.update(case.pop("setenv", {}))  # read by the library at its first table build
     fn = {"solve": solve, "iterate": iterate, "plan": plan, "batch": batch,
           "adjoint": adjoint, "batch_adjoint": batch_adjoint, "gen": gen, "analyze": analyze,
-          "identify": identify, "plan_freq": plan_freq}[case.pop("kind")]
+          "identify": identify, "plan_freq": plan_freq,
+          "plan_freq_first": plan_freq_first}[case.pop("kind")]
     print("RESULT " + json.dumps(fn(**case)), flush=True)

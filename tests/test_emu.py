@@ -50,6 +50,9 @@ CASES = {
     "plan": dict(kind="plan", n=4096, bins=101, bits=5, seed=1),
     "plan_four_step": dict(kind="plan", n=1 << 16, bins=4097, bits=4, seed=2),
     "plan_freq": dict(kind="plan_freq", n=1 << 14, bins=301, bits=6, m=900, seed=4),
+    # device memory that starts as large integers, and fills that return early
+    "plan_freq_first": dict(kind="plan_freq_first", n=1 << 14, bins=101, bits=8, m=50, seed=6,
+                            setenv={"EMU_GARBAGE": "0x7f", "EMU_LATE_FILL": "1"}),
     "iterate_four_step": dict(kind="iterate", n=1 << 16, k=2100, sigma=1e-6, seed=3, bins=4201),
     "solve_0": dict(kind="solve", n=1 << 14, k=20, sigma=1e-6, seed=7, precision=0, repeat=2),
     "solve_1": dict(kind="solve", n=1 << 14, k=20, sigma=3e-6, seed=7, precision=1, repeat=2),
@@ -114,6 +117,13 @@ def test_emu_plan_bin_in_freq_exact_sums(emu_runs):
     another order."""
     r = result(emu_runs, "plan_freq")
     assert r["abs_err"] < 1e-12 * r["scale"] and r["identical"], r
+
+
+def test_emu_bin_in_freq_first_call(emu_runs):
+    """A plan's first BinInFreq, on a non-blocking stream: nothing of it rests
+    on a fill of the plan's scratch that its creation did not wait for."""
+    r = result(emu_runs, "plan_freq_first")
+    assert r["abs_err"] < 1e-12 * r["scale"], r
 
 
 def test_emu_iterate_four_step_with_found_modes(emu_runs):

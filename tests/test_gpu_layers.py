@@ -1,5 +1,7 @@
 """The layers' kernels at the edges of their tiles and launches, against the
 CPU oracle (1e-12 of the largest value, as in the parity tests)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -32,6 +34,29 @@ def test_bin_in_freq_edges(gpu, orc, n, bins, m):
         orc.bin_in_freq(keys.astype(np.int32), coefs, n, bins, 1e-6, bits, tf_o, 77, ref, version=1)
         plan.bin_in_freq(keys, coefs, tf, 77, got)
         assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
+
+
+# the second: more modes than the exponent pass has threads, more sums too
+@pytest.mark.parametrize("n,bins,m", [(1 << 14, 101, 50), (1 << 18, 4095, 140000)])
+def test_bin_in_freq_first_call_on_a_stream(gpu, orc, n, bins, m):
+    """A fresh plan's first BinInFreq on a non-blocking stream."""
+    rng = np.random.default_rng(m)
+    bits = orc.num_bits(n, bins)
+    tf_o, tf = _tf(gpu, orc, n, m)
+    keys = rng.choice(n, m, replace=False).astype(np.int64)
+    coefs = rng.standard_normal(m) + 1j * rng.standard_normal(m)
+    base = rng.standard_normal((1 + 2 * bits, bins)) + 1j
+    ref = base.copy()
+    orc.bin_in_freq(keys.astype(np.int32), coefs, n, bins, 1e-6, bits, tf_o, 77, ref, version=1)
+    stream = C.c_void_p()
+    assert gpu.lib().mpsft_stream_create(C.byref(stream)) == 0
+    kd, cd, od = (gpu.DeviceArray.from_numpy(v) for v in (keys, coefs, base))
+    plan = gpu.Plan(n, bins, 1e-6, bits)
+    plan.bin_in_freq_dev(kd, cd, m, tf, 77, od, stream)
+    assert gpu.lib().mpsft_stream_synchronize(stream) == 0
+    got = od.to_numpy(np.complex128, base.shape)
+    assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
+    assert gpu.lib().mpsft_stream_destroy(stream) == 0
 
 
 def test_iterate_after_overflow_changes_nothing(gpu):
