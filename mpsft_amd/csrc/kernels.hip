@@ -2397,7 +2397,8 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
 // the threads: a pass for the grid exponent, a pass adding the limbs into
 // limbs[(row B + bin) kLimbs ...], and one subtracting each bin's sum.  Each
 // pass writes the scratch that the next one reads, so a call depends on
-// nothing that was in it before.
+// nothing that was in it before.  The sums hold finite terms: a component
+// that is not finite goes straight to its bin, which it alone decides.
 //
 // Bound by latency: a term costs two erf and two sincospi, 2 x 4 integer
 // atomics follow, and there are few modes.  So a thread takes one (mode,
@@ -2434,9 +2435,17 @@ __device__ __forceinline__ int32_t BlockMax(int32_t e) {
   return e;
 }
 
-// limbs[0..count) = 0 (a kernel rather than a memset), and emax[blockIdx.x] =
-// the exponent of the workgroup's largest |coef| wf (kNoTerms if all are 0).
+// |v| < 2^TermExponent(v), or kNoTerms: a mode of which nothing goes to the
+// sums (zero, or a component that is not finite).
 constexpr int32_t kNoTerms = -(1 << 30);
+__device__ __forceinline__ int32_t TermExponent(double2 v) {
+  const double h = hypot(v.x, v.y);
+  if (isfinite(h)) return h > 0.0 ? ilogb(h) + 1 : kNoTerms;
+  return isfinite(v.x) && isfinite(v.y) ? 1025 : kNoTerms;  // h passed the largest double
+}
+
+// limbs[0..count) = 0 (a kernel rather than a memset), and emax[blockIdx.x] =
+// the largest exponent of the workgroup's modes.
 __global__ void __launch_bounds__(kThreads)
     k_freq_direct_max(int64_t n, int64_t mask, BParams bp, DevTf tf, const int64_t *k0s,
                       const double2 *coefs, int64_t m, int32_t *emax, unsigned long long *limbs,
@@ -2444,12 +2453,10 @@ __global__ void __launch_bounds__(kThreads)
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t gsize = int64_t(gridDim.x) * blockDim.x;
   for (int64_t j = i; j < count; j += gsize) limbs[j] = 0ull;
-  double mx = 0.0;
-  for (int64_t j = i; j < m; j += gsize) {
-    const DirectMode d = DirectBase(n, mask, bp, tf, k0s[j], coefs[j]);
-    mx = fmax(mx, hypot(d.cw.x, d.cw.y));
-  }
-  const int32_t e = BlockMax(mx > 0.0 ? ilogb(mx) + 1 : kNoTerms);
+  int32_t e = kNoTerms;
+  for (int64_t j = i; j < m; j += gsize)
+    e = max(e, TermExponent(DirectBase(n, mask, bp, tf, k0s[j], coefs[j]).cw));
+  e = BlockMax(e);
   if (threadIdx.x == 0) emax[blockIdx.x] = e;
 }
 
@@ -2463,12 +2470,26 @@ __device__ __forceinline__ TermGrid TermGridOf(int32_t e) {
   return g;
 }
 
+// Term v of bin j: into the sums, or out of them where it is not finite.
+__device__ __forceinline__ void DirectAdd(unsigned long long *limbs, double2 *out, int64_t j,
+                                          double2 v, const TermGrid &g) {
+  if (!isfinite(v.x)) {
+    atomicAdd(&out[j].x, -v.x);
+    v.x = 0.0;
+  }
+  if (!isfinite(v.y)) {
+    atomicAdd(&out[j].y, -v.y);
+    v.y = 0.0;
+  }
+  if (g.any) LimbAdd(limbs + kLimbs * j, 1, v, g);
+}
+
 // One (mode, bit) per thread.  emax: the first pass's `slots` exponents;
 // their largest goes to emax[kFreqSlots], for the last pass.
 __global__ void __launch_bounds__(kThreads)
     k_freq_direct_add(int64_t n, int64_t mask, BParams bp, DevTf tf, int64_t q,
                       const int64_t *k0s, const double2 *coefs, int64_t m, int32_t *emax,
-                      int32_t slots, unsigned long long *limbs) {
+                      int32_t slots, unsigned long long *limbs, double2 *out) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   int32_t e = kNoTerms;
   for (int32_t k = threadIdx.x; k < slots; k += kThreads) e = max(e, emax[k]);
@@ -2476,7 +2497,6 @@ __global__ void __launch_bounds__(kThreads)
   if (i == 0) emax[kFreqSlots] = e;
   const TermGrid g = TermGridOf(e);
   const int64_t work = m * bp.bits;
-  if (!g.any) return;
   for (int64_t j = i; j < work; j += int64_t(gridDim.x) * blockDim.x) {
     // modes over the lanes (coalesced reads), bits over the blocks
     const int32_t bit = int32_t(j / m);
@@ -2484,10 +2504,10 @@ __global__ void __launch_bounds__(kThreads)
     const DirectMode d = DirectBase(n, mask, bp, tf, k0s[mi], coefs[mi]);
     const double2 base = Cmul(d.cw, CisFrac(ModN(q * d.k1 + tf.c * d.k0, n, mask), n));
     const double2 t = CisFrac(ModN((int64_t(bp.B) << bit) * d.k1, n, mask), n);
-    unsigned long long *acc = limbs + kLimbs * (int64_t(2 * bit + 1) * bp.B + d.bin);
-    if (bit == 0) LimbAdd(limbs + kLimbs * int64_t(d.bin), 1, base, g);
-    LimbAdd(acc, 1, Cmul(base, t), g);
-    LimbAdd(acc + kLimbs * int64_t(bp.B), 1, Cmul(base, Conj(t)), g);
+    const int64_t at = int64_t(2 * bit + 1) * bp.B + d.bin;
+    if (bit == 0) DirectAdd(limbs, out, d.bin, base, g);
+    DirectAdd(limbs, out, at, Cmul(base, t), g);
+    DirectAdd(limbs, out, at + bp.B, Cmul(base, Conj(t)), g);
   }
 }
 
@@ -3548,7 +3568,7 @@ hipError_t LaunchBinInFreqDirect(int64_t n, int64_t mask, const BParams &bp,
   hipLaunchKernelGGL(k_freq_direct_max, dim3(slots), dim3(kThreads), 0, s, n, mask, bp, tf, k0, coef,
                      m, emax, limbs, kLimbs * bins);
   hipLaunchKernelGGL(k_freq_direct_add, dim3(Blocks(m * bp.bits)), dim3(kThreads), 0, s, n, mask, bp,
-                     tf, q, k0, coef, m, emax, slots, limbs);
+                     tf, q, k0, coef, m, emax, slots, limbs, out);
   hipLaunchKernelGGL(k_freq_direct_sub, dim3(Blocks(bins)), dim3(kThreads), 0, s, limbs, emax, bins,
                      out);
   return hipGetLastError();

@@ -47,6 +47,7 @@ inline int2 make_int2(int x, int y) { return int2{x, y}; }
 inline double2 make_double2(double x, double y) { return double2{x, y}; }
 inline float2 make_float2(float x, float y) { return float2{x, y}; }
 
+using std::isfinite;
 using std::max;
 using std::min;
 

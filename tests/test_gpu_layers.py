@@ -59,6 +59,36 @@ def test_bin_in_freq_first_call_on_a_stream(gpu, orc, n, bins, m):
     assert gpu.lib().mpsft_stream_destroy(stream) == 0
 
 
+@pytest.mark.parametrize("special", [np.inf, np.nan, 1.3e308 * (1 + 1j)])
+def test_bin_in_freq_beyond_the_finite(gpu, orc, special):
+    """A coefficient that is not finite, or whose modulus is not: its own bins
+    are as the oracle's (finite or not), and the others' sums are right."""
+    n, bins, m = 1 << 14, 301, 40
+    rng = np.random.default_rng(3)
+    bits = orc.num_bits(n, bins)
+    tf_o, tf = _tf(gpu, orc, n, 21)
+    keys = rng.choice(n, m, replace=False).astype(np.int64)
+    coefs = rng.standard_normal(m) + 1j * rng.standard_normal(m)
+    # the mode nearest a bin's centre, where the window is 1
+    k1 = (int(tf_o[0]) * keys + int(tf_o[1])) % n
+    at = int(np.argmin(np.abs((k1 * bins / n) % 1 - 0.5)))
+    coefs[at] = special
+    base = rng.standard_normal((1 + 2 * bits, bins)) + 1j
+    ref, got = base.copy(), base.copy()
+    orc.bin_in_freq(keys.astype(np.int32), coefs, n, bins, 1e-6, bits, tf_o, 77, ref, version=1)
+    gpu.Plan(n, bins, 1e-6, bits).bin_in_freq(keys, coefs, tf, 77, got)
+    own = np.arange(bins) == k1[at] * bins // n
+    # beside a term of 2^1025 the sums resolve 2^-94 of it
+    tol = TOL * np.abs(ref[:, ~own]).max() if not np.isfinite(special) else 2.0 ** (1025 - 94) * m
+    assert np.abs(got[:, ~own] - ref[:, ~own]).max() <= tol
+    a, b = (np.concatenate([v[:, own].real, v[:, own].imag]) for v in (got, ref))
+    # on the edge of the range the oracle's products may pass it where ours do not
+    assert (np.isfinite(a) == np.isfinite(b)).mean() >= 0.9
+    both = np.isfinite(a) & np.isfinite(b)
+    assert (np.abs(a[both] / 1e308 - b[both] / 1e308) <= TOL).all()
+    assert both.any() == np.isfinite(special)
+
+
 def test_iterate_after_overflow_changes_nothing(gpu):
     """A map that overflowed its capacity stays as it is: the one-launch
     parameters of Iterate carry the stop to the later kernels."""
