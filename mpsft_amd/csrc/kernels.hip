@@ -109,10 +109,12 @@ __device__ __forceinline__ double2 LoadX(const double2 *p) {
 }
 __device__ __forceinline__ double2 Widen(float2 v) { return make_double2(double(v.x), double(v.y)); }
 
-// A value at a wavefront-uniform address that this launch writes no byte of,
-// by scalar loads: it and what is computed from it alone stay in SGPRs.  Read
-// plainly, a batch's Ctx and IterParams (whose memory the compiler must
-// assume the kernel writes) sit in VGPRs, one copy per lane.
+// A value at a wavefront-uniform address of device memory (never a kernel
+// parameter's or LDS) that this launch writes no byte of, by scalar loads: it
+// and what is computed from it alone stay in SGPRs.  Read plainly, a batch's
+// Ctx and IterParams (whose memory the compiler must assume the kernel
+// writes) sit in VGPRs, one copy per lane.  The emulator of the CPU tests
+// checks both conditions on every launch.
 typedef const uint32_t __attribute__((address_space(4))) *ConstU32;
 template <typename T>
 __device__ __forceinline__ T LoadUniform(const T *p) {
@@ -623,11 +625,10 @@ struct Lags {
 // Workgroups below kPrepBlocks instead compute the BinInFreq terms of every
 // found mode for this iteration.
 // blk: this workgroup's block index within the signal's launch.
-// x, qs: the signal and the iteration's q per trial.
-template <typename Tx, bool kNt = true, bool kSort = false>
+// xv: the signal; q_of(trial): the iteration's q of a trial.
+template <typename Tx, bool kNt = true, bool kSort = false, typename QOf>
 __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, const void *xv,
-                                         const int64_t *qs, int32_t trials, int32_t tile,
-                                         double2 *lds);
+                                         QOf q_of, int32_t trials, int32_t tile, double2 *lds);
 
 // The BinInFreq factor of mode k0 (k1 = its image under the transform) in
 // row 0 for offset q: wf(xi) e^{2 pi i (q k1 + c k0)/n}, and its bin.  Every
@@ -686,6 +687,13 @@ __device__ __forceinline__ void FreqTerms(const Ctx &c, const IterParams &ip, co
 __device__ __forceinline__ const int64_t *IterQs(const Ctx &c, int32_t it) {
   return c.qs + int64_t(it) * c.trials_cap;
 }
+// One of them, for a trial that every lane shares.
+struct UniformQ {
+  const int64_t *qs;
+  __device__ __forceinline__ int64_t operator()(int32_t trial) const {
+    return LoadUniform(qs + trial);
+  }
+};
 
 template <typename Tx>
 __device__ __forceinline__ void BinTimeBody(const Ctx &c, int p, int blk, double2 *lds) {
@@ -699,7 +707,7 @@ __device__ __forceinline__ void BinTimeBody(const Ctx &c, int p, int blk, double
   if (blk < kPrepBlocks)
     FreqTerms(c, ip, qs, fx.trials, blk, kPrepBlocks);
   else
-    TileFold<Tx>(c, ip, fx.x, qs, fx.trials, blk - kPrepBlocks, lds);
+    TileFold<Tx>(c, ip, fx.x, UniformQ{qs}, fx.trials, blk - kPrepBlocks, lds);
 }
 
 // The lags of a tile in buckets of increasing position a B lambda mod n (n =
@@ -751,10 +759,9 @@ __device__ __forceinline__ void SortLags(const Lags &L, uint32_t aB, uint32_t m3
 // The gather-fold of one tile (trial, block of R residues) of an iteration
 // with parameters ip (see BinTimeBody).  kSort: the sorted order is compiled
 // in (and taken where ip.sorted is set).
-template <typename Tx, bool kNt, bool kSort>
+template <typename Tx, bool kNt, bool kSort, typename QOf>
 __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, const void *xv,
-                                         const int64_t *qs, int32_t trials, int32_t tile,
-                                         double2 *lds) {
+                                         QOf q_of, int32_t trials, int32_t tile, double2 *lds) {
   const int32_t B = ip.B, f = ip.f, bits = ip.bits, p2 = ip.p2, rows = ip.rows;
   const DevTf tf = ip.tf;
   const int64_t n = c.n, mask = c.mask;
@@ -768,7 +775,7 @@ __device__ __forceinline__ void TileFold(const Ctx &c, const IterParams &ip, con
   const int32_t rho0 = (tile - trial * nblk) * R;
   const int32_t nrho = min(R, B - rho0);
   const Lags L(bits, f);
-  const int64_t q = LoadUniform(qs + trial);
+  const int64_t q = q_of(trial);
   const Tx *x = static_cast<const Tx *>(xv);
 
   // [nlam][R] samples as stored in x (complex64 samples take half the LDS
@@ -955,7 +962,9 @@ __global__ void __launch_bounds__(kThreads) k_bin_time_once(Ctx c, OneShot o) {
   if (blk < kPrepBlocks)
     FreqTerms(c, ip, o.q, o.trials, blk, kPrepBlocks);
   else
-    TileFold<Tx>(c, ip, o.x, o.q, o.trials, blk - kPrepBlocks, lds);
+    // (o.q by plain loads: a parameter's address is not constant memory's)
+    TileFold<Tx>(c, ip, o.x, [&](int32_t trial) { return o.q[trial]; }, o.trials,
+                 blk - kPrepBlocks, lds);
 }
 
 __global__ void k_publish_once(Ctx c, OneShot o, IdOut out, IdOut *idout) {
@@ -2214,7 +2223,7 @@ __global__ void __launch_bounds__(kThreads)
     }
     return;
   }
-  TileFold<Tx>(c, ip, fx.x, IterQs(c, ip.it), trials, pb - kPrepBlocks, lds);
+  TileFold<Tx>(c, ip, fx.x, UniformQ{IterQs(c, ip.it)}, trials, pb - kPrepBlocks, lds);
 }
 
 template <int kPaths>
@@ -2728,7 +2737,7 @@ __device__ __forceinline__ void BinTimeUnit(const Ctx &c, int p, int32_t unit, d
   if (unit < nprep)
     FreqTerms(c, ip, qs, trials, unit, nprep);
   else
-    TileFold<Tx, false, true>(c, ip, LoadUniform(&st->x), qs, trials, unit - nprep, lds);
+    TileFold<Tx, false, true>(c, ip, LoadUniform(&st->x), UniformQ{qs}, trials, unit - nprep, lds);
 }
 
 template <typename Tx>

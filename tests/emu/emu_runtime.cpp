@@ -13,6 +13,7 @@
 #include <map>
 #include <mutex>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 namespace emu {
@@ -122,7 +123,10 @@ void Trampoline() {
   setcontext(&S->main);
 }
 
+std::unordered_map<const uint32_t *, uint32_t> constants;  // the launch's constant words
+
 void Run(const Node &nd) {
+  constants.clear();
   if (nd.block.x == 0 || nd.block.x > 1024 || nd.block.y != 1 || nd.block.z != 1 ||
       nd.grid.y != 1 || nd.grid.z != 1) {
     std::fprintf(stderr, "emu: unsupported launch shape\n");
@@ -178,6 +182,11 @@ void Run(const Node &nd) {
     std::free(blk.lds);
   }
   sched = nullptr;
+  for (const auto &w : constants)
+    if (*w.first != w.second) {
+      std::fprintf(stderr, "emu: a launch changed a word that it read as constant\n");
+      std::abort();
+    }
 }
 
 }  // namespace
@@ -333,6 +342,17 @@ Device &Dev() {
   return *d;
 }
 }  // namespace
+
+uint32_t emu::ConstantWord(const uint32_t *p) {
+  if (tid.x == 0) {  // the address is the same for every thread
+    if (!Tracked(p)) {
+      std::fprintf(stderr, "emu: constant load outside device memory\n");
+      std::abort();
+    }
+    constants.emplace(p, *p);
+  }
+  return *p;
+}
 
 void emu::Launch(void *stream, dim3 grid, dim3 block, size_t lds, std::function<void()> body) {
   Node nd{grid, block, lds, std::move(body)};

@@ -63,6 +63,18 @@ double ShflD(double v, int src);
 int ShflI(int v, int src);
 uint64_t Ballot(int pred);
 void Launch(void *stream, dim3 grid, dim3 block, size_t lds, std::function<void()> body);
+
+// What kernels.hip's pointers to constant memory become here (see the
+// Makefile): words of device memory that the launch does not change.  A word
+// elsewhere (a kernel argument's private copy, LDS) ends the process, and so
+// does one whose value at the launch's end is another.
+uint32_t ConstantWord(const uint32_t *p);
+struct ConstantWords {
+  const uint32_t *p;
+  template <typename T>
+  explicit ConstantWords(const T *q) : p(reinterpret_cast<const uint32_t *>(q)) {}
+  uint32_t operator[](size_t i) const { return ConstantWord(p + i); }
+};
 }  // namespace emu
 
 #define threadIdx emu::tid
