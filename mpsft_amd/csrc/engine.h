@@ -114,8 +114,9 @@ struct IdOut {
 // The parameters of one iteration.  Every k_bin_time workgroup derives them
 // from the previous iteration's slot and the counters k_identify left;
 // workgroup 0 publishes them in slot (iteration & 1) for the iteration's
-// k_bin_fft and k_identify.
-struct IterParams {
+// k_bin_fft and k_identify.  IterFixed are the fields that k_late_fft loads
+// as constant while its first workgroup stores `done`.
+struct IterFixed {
   DevTf tf;
   int64_t q[kMaxTrials];
   int64_t tab_off;
@@ -123,7 +124,9 @@ struct IterParams {
   double bin_thr, sv_thr;
   int32_t B, bits, rows, f, P, p2, M, logM, R;
   int32_t G, sorted, slices, slice_shift;  // as BParams
-  int32_t it;    // iteration index
+  int32_t it;  // iteration index
+};
+struct IterParams : IterFixed {
   int32_t done;  // the loop stopped before this iteration
 };
 

@@ -2274,8 +2274,9 @@ __global__ void __launch_bounds__(kFftThreads) k_late_fft(Ctx c, int p) {
     if (c.progress && lc.done) PublishStop(c, lc.it, lc.stale, flags, count);
   }
   if (done) return;
-  // (the launch writes P[p].done, which is not read from here on)
-  const IterParams ip = LoadUniform(&st->P[p]);
+  IterParams ip;  // without P[p].done, which workgroup 0 has just stored
+  static_cast<IterFixed &>(ip) = LoadUniform(static_cast<const IterFixed *>(&st->P[p]));
+  ip.done = 0;
   const int32_t trials = fx.trials, rows = ip.rows;
   const int32_t trial = blockIdx.x / c.rows_cap;
   const int32_t row = blockIdx.x - trial * c.rows_cap;
