@@ -376,6 +376,7 @@ Engine::~Engine() {
   if (p_tfs_) (void)hipHostFree(p_tfs_);
   if (p_qs_) (void)hipHostFree(p_qs_);
   if (h_progress_) (void)hipHostFree(const_cast<int32_t *>(h_progress_));
+  if (tail_ev_) (void)hipEventDestroy(tail_ev_);
 }
 
 // The gather-fold's tiles of one B.  G is the default width, so that a
@@ -850,7 +851,23 @@ int Engine::EnsureGraph(int32_t iters, hipStream_t s) {
 // changes buffers or launches on another stream does so first.
 void Engine::Drain() {
   if (!tail_pending_) return;
-  (void)hipStreamSynchronize(tail_stream_);
+  if (tail_stream_)
+    (void)hipEventSynchronize(tail_ev_);
+  else
+    (void)hipStreamSynchronize(nullptr);
+  tail_pending_ = false;
+}
+
+// Marks the end of the launches a solve leaves queued on s (the null stream
+// outlives the engine and needs no mark).
+void Engine::LeaveTail(hipStream_t s) {
+  tail_pending_ = true;
+  tail_stream_ = s;
+  if (!s) return;
+  if ((tail_ev_ || hipEventCreateWithFlags(&tail_ev_, hipEventDisableTiming) == hipSuccess) &&
+      hipEventRecord(tail_ev_, s) == hipSuccess)
+    return;
+  (void)hipStreamSynchronize(s);
   tail_pending_ = false;
 }
 
@@ -1072,8 +1089,7 @@ int Engine::Solve(const void *x, const mpsft_solve_options &opt, uint32_t seed,
       // The device reported the stop and its result in pinned memory.  The
       // launches queued past the stop exit at once without touching the
       // results; the next call that needs them idle waits (Drain).
-      tail_pending_ = true;
-      tail_stream_ = s;
+      LeaveTail(s);
       h_state_->L[0].done = 1;
       h_state_->iters = h_progress_[3];
       h_state_->stop_stale = h_progress_[4];
@@ -1411,7 +1427,8 @@ int Engine::ModesCount(int64_t *count) {
 }
 
 // One kernel lays keys and coefficients out side by side and one copy brings
-// them to the host, in stream order behind the launches a solve left queued.
+// them to the host, both on the null stream: behind the launches that a solve
+// there left queued, and after waiting for those it left on another stream.
 // (Two state reads, then a launch and two copies, each waited for, made a
 // solve of n = 2^16, S = 60 with its modes 285 us; it is 237 now.)
 int Engine::ModesGet(int64_t *keys, double *coefs, int64_t cap, int64_t *count) {
@@ -1421,11 +1438,12 @@ int Engine::ModesGet(int64_t *keys, double *coefs, int64_t cap, int64_t *count) 
   *count = m;
   if (cap < m) return MPSFT_ERR_SHAPE;
   if (m == 0) return MPSFT_OK;
-  const hipStream_t s = tail_pending_ ? tail_stream_ : nullptr;
-  HIP_OK(LaunchGetModes(MakeCtx(), d_tmp_, m, s));
+  if (tail_stream_) Drain();
+  HIP_OK(LaunchGetModes(MakeCtx(), d_tmp_, m, nullptr));
   modes_host_.resize(size_t(m) * kModeBytes);
-  HIP_OK(hipMemcpyAsync(modes_host_.data(), d_tmp_, modes_host_.size(), hipMemcpyDeviceToHost, s));
-  HIP_OK(hipStreamSynchronize(s));
+  HIP_OK(hipMemcpyAsync(modes_host_.data(), d_tmp_, modes_host_.size(), hipMemcpyDeviceToHost,
+                        nullptr));
+  HIP_OK(hipStreamSynchronize(nullptr));
   tail_pending_ = false;
   std::memcpy(coefs, modes_host_.data(), size_t(m) * sizeof(double2));
   std::memcpy(keys, modes_host_.data() + size_t(m) * sizeof(double2), size_t(m) * sizeof(int64_t));

@@ -416,9 +416,13 @@ class Engine {
   int32_t rec_iters_ = 0;
   int64_t rec_id_ = 0;
 
-  // launches a solve left queued past its stop, on tail_stream_
+  // launches a solve left queued past its stop, on tail_stream_.  A caller's
+  // stream may be destroyed once the solve has returned: its handle is only
+  // compared after that, and the launches are waited for by tail_ev_.
   bool tail_pending_ = false;
   hipStream_t tail_stream_ = nullptr;
+  hipEvent_t tail_ev_ = nullptr;
+  void LeaveTail(hipStream_t s);
   void Drain();
   // PrepareSolve's key: the options, buffer shapes and table contents of
   // the last full preparation

@@ -12,6 +12,7 @@
 #include <deque>
 #include <map>
 #include <mutex>
+#include <set>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -354,16 +355,37 @@ uint32_t emu::ConstantWord(const uint32_t *p) {
   return *p;
 }
 
+namespace {
+// Streams that exist; a call on any other (but the null stream) fails, and
+// hipGetLastError reports it once.
+std::mutex g_stream_mu;
+std::set<hipStream_t> g_streams;
+thread_local hipError_t g_last_error = hipSuccess;
+
+bool Live(hipStream_t s) {
+  if (!s) return true;
+  std::lock_guard<std::mutex> lk(g_stream_mu);
+  if (g_streams.count(s)) return true;
+  g_last_error = hipErrorContextIsDestroyed;
+  return false;
+}
+}  // namespace
+
 void emu::Launch(void *stream, dim3 grid, dim3 block, size_t lds, std::function<void()> body) {
   Node nd{grid, block, lds, std::move(body)};
   if (g_capture && static_cast<void *>(g_capture_stream) == stream) {
     g_capture->nodes.push_back(std::move(nd));
     return;
   }
+  if (!Live(static_cast<hipStream_t>(stream))) return;
   Dev().Submit([nd = std::move(nd)] { Run(nd); });
 }
 
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last_error;
+  g_last_error = hipSuccess;
+  return e;
+}
 hipError_t hipGetDeviceCount(int *count) {
   *count = 1;
   return hipSuccess;
@@ -403,8 +425,9 @@ hipError_t hipMemcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind) {
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind k,
-                          hipStream_t) {
+                          hipStream_t s) {
   if (g_capture) return hipErrorNotSupported;
+  if (!Live(s)) return hipErrorContextIsDestroyed;
   if (Tracked(dst) && Tracked(src)) {
     if (bytes) Dev().Submit([=] { std::memcpy(dst, src, bytes); });
     return hipSuccess;
@@ -442,15 +465,23 @@ hipError_t hipDeviceSynchronize() {
 }
 hipError_t hipStreamCreate(hipStream_t *s) {
   *s = new EmuStream{0};
+  std::lock_guard<std::mutex> lk(g_stream_mu);
+  g_streams.insert(*s);
   return hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return hipStreamCreate(s); }
 hipError_t hipStreamDestroy(hipStream_t s) {
   Dev().Wait();
+  if (!s || !Live(s)) return hipErrorContextIsDestroyed;
+  {
+    std::lock_guard<std::mutex> lk(g_stream_mu);
+    g_streams.erase(s);
+  }
   delete s;
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (!Live(s)) return hipErrorContextIsDestroyed;
   Dev().Wait();
   if (!s) RunLateFills();
   return hipSuccess;
@@ -481,7 +512,8 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
   delete e;
   return hipSuccess;
 }
-hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s) {
+  if (!Live(s)) return hipErrorContextIsDestroyed;
   for (const auto &nd : e->nodes) Dev().Submit([nd] { emu::Run(nd); });
   return hipSuccess;
 }
@@ -489,12 +521,14 @@ hipError_t hipEventCreate(hipEvent_t *e) {
   *e = new EmuEvent;
   return hipSuccess;
 }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) {
   Dev().Wait();
   delete e;
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  if (!Live(s)) return hipErrorContextIsDestroyed;
   Dev().Submit([e] { e->t = std::chrono::steady_clock::now(); });
   return hipSuccess;
 }

@@ -150,6 +150,7 @@ enum : int {
   hipSuccess = 0,
   hipErrorInvalidValue = 1,
   hipErrorOutOfMemory = 2,
+  hipErrorContextIsDestroyed = 709,
   hipErrorNotSupported = 801,
 };
 enum hipMemcpyKind {
@@ -209,7 +210,9 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t g, hipGraphNode_t *
 hipError_t hipGraphDestroy(hipGraph_t g);
 hipError_t hipGraphExecDestroy(hipGraphExec_t e);
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s);
+constexpr unsigned hipEventDisableTiming = 2;
 hipError_t hipEventCreate(hipEvent_t *e);
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned flags);
 hipError_t hipEventDestroy(hipEvent_t e);
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s);
 hipError_t hipEventSynchronize(hipEvent_t e);

@@ -60,6 +60,29 @@ def solve(n, k, sigma, seed, precision=0, repeat=1, x_path=None, **kw):
     return out
 
 
+def stream_ends(n, k, sigma, seed):
+    """Solves on streams that are destroyed before the next call."""
+    s = gpu.Solver(n, gpu.solve_options(k, sigma))
+    xd = s.upload(signal(n, k, sigma, seed))
+    s.solve(xd, seed)
+    want = s.modes_dict()
+    same = []
+    for after in ("modes", "solve", "set_modes", "log"):
+        stream = C.c_void_p()
+        gpu.lib().mpsft_stream_create(C.byref(stream))
+        s.solve(xd, seed, stream=stream)
+        gpu.lib().mpsft_stream_destroy(stream)
+        if after == "solve":
+            s.solve(xd, seed)
+        elif after == "set_modes":
+            s.set_modes({})
+            s.set_modes(want)
+        elif after == "log":
+            s.log()
+        same.append(s.modes_dict() == want)
+    return dict(same=same, n_found=len(want))
+
+
 def iterate(n, k, sigma, seed, bins, steps=2):
     x = signal(n, k, sigma, seed)
     kw = dict(bins=bins, window_delta=1e-6, trials=1, bin_threshold=3 * sigma / np.sqrt(bins),
@@ -296,5 +319,5 @@ if __name__ == "__main__":
     fn = {"solve": solve, "iterate": iterate, "plan": plan, "batch": batch,
           "adjoint": adjoint, "batch_adjoint": batch_adjoint, "gen": gen, "analyze": analyze,
           "identify": identify, "plan_freq": plan_freq,
-          "plan_freq_first": plan_freq_first}[case.pop("kind")]
+          "plan_freq_first": plan_freq_first, "stream_ends": stream_ends}[case.pop("kind")]
     print("RESULT " + json.dumps(fn(**case)), flush=True)

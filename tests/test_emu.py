@@ -54,6 +54,7 @@ CASES = {
     "plan_freq_first": dict(kind="plan_freq_first", n=1 << 14, bins=101, bits=8, m=50, seed=6,
                             setenv={"EMU_GARBAGE": "0x7f", "EMU_LATE_FILL": "1"}),
     "iterate_four_step": dict(kind="iterate", n=1 << 16, k=2100, sigma=1e-6, seed=3, bins=4201),
+    "stream_ends": dict(kind="stream_ends", n=1 << 14, k=20, sigma=1e-6, seed=7),
     "solve_0": dict(kind="solve", n=1 << 14, k=20, sigma=1e-6, seed=7, precision=0, repeat=2),
     "solve_1": dict(kind="solve", n=1 << 14, k=20, sigma=3e-6, seed=7, precision=1, repeat=2),
     "solve_2": dict(kind="solve", n=1 << 16, k=300, sigma=1e-6, seed=5, precision=0, repeat=1),
@@ -147,6 +148,13 @@ def test_emu_solve_graph(emu_runs, case):
     assert r["back_to_back_iters"] == [r["iters0"]] * 3 and r["back_to_back_same"]
     assert r["bins"] == r["ref_bins"] and r["same_support"]
     assert r["max_rel_err"] < 1e-10
+
+
+def test_emu_modes_after_the_stream_ends(emu_runs):
+    """A solve's stream may be destroyed once the solve has returned: the modes
+    and the next calls are as after a solve on the null stream."""
+    r = result(emu_runs, "stream_ends")
+    assert r["n_found"] == 20 and r["same"] == [True] * 4, r
 
 
 def test_emu_sliced_gather_fold(emu_runs):

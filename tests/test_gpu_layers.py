@@ -208,6 +208,24 @@ def test_mode_counts_follow_every_call(gpu):
     assert sizes == [len(maps[0]), len(maps[1])]
 
 
+def test_modes_after_the_stream_ends(gpu):
+    """A solve's stream may be destroyed once the solve has returned."""
+    from mpsft_amd.signals import make_signal
+    n, k = 1 << 16, 60
+    s = gpu.Solver(n, gpu.solve_options(k, 1e-6))
+    xd = s.upload(make_signal(n, k, 1e-6, seed=3)[0])
+    s.solve(xd, 4)
+    want = s.modes_dict()
+    for _ in range(3):
+        stream = C.c_void_p()
+        assert gpu.lib().mpsft_stream_create(C.byref(stream)) == 0
+        s.solve(xd, 4, stream=stream)
+        assert gpu.lib().mpsft_stream_destroy(stream) == 0
+        assert s.modes_dict() == want
+    s.solve(xd, 4)
+    assert s.modes_dict() == want
+
+
 @pytest.mark.parametrize("n,k,min_bins,precision", [
     (1 << 16, 50, 101, 0),  # 2^(bits-1) B + f B below n: offsets have one positive lag
     (1 << 16, 50, 127, 0),  # above n: offsets below f B have two
