@@ -928,7 +928,6 @@ int Engine::PrepareSolve(const void *x, const mpsft_solve_options &opt, uint32_t
   a->min_bins = opt.min_bins;
   a->max_stale = opt.max_stale_iter;
   a->max_iter = max_iter;
-  a->bits_override = 0;
   a->win_thr = opt.window_threshold;
   return MPSFT_OK;
 }

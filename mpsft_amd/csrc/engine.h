@@ -151,8 +151,8 @@ struct LoopCounters {
 // The part of the loop state that is fixed for a call.
 struct DevFixed {
   const void *x;  // input signal (double2 or float2)
-  int32_t mode, trials, k, min_bins, max_stale, max_iter, bits_override, B_fixed;
-  double win_thr, bin_thr_fixed, sv_thr_fixed;
+  int32_t mode, trials, k, min_bins, max_stale, max_iter;
+  double win_thr;
 };
 
 // Device-resident loop state.

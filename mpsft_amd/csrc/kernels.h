@@ -5,16 +5,14 @@
 
 namespace mpsft {
 
-// Initial loop state for k_init.
+// Initial loop state of a solve or a replay (k_init, k_reset).
 struct InitArgs {
   const void *x;
-  int32_t mode;
-  int32_t B;          // bins for Iterate / BinInTime (the solve derives its own)
+  int32_t mode;  // kModeSolve or kModeReplay
+  int32_t B;     // first bins
   int32_t trials;
   int32_t k, min_bins, max_stale, max_iter;
-  int32_t bits_override;  // > 0: use this bits instead of the table's
-  int32_t keep_modes;     // 1: keep the found-mode map (Iterate)
-  double bin_thr, sv_thr, win_thr;
+  double win_thr;
 };
 
 // One iteration with explicit parameters (a plan call or Iterate), passed to

@@ -380,15 +380,9 @@ __device__ __forceinline__ void InitBody(const Ctx &c, const InitArgs &a) {
   st->min_bins = a.min_bins;
   st->max_stale = a.max_stale;
   st->max_iter = a.max_iter;
-  st->bits_override = a.bits_override;
-  st->B_fixed = a.B;
   st->win_thr = a.win_thr;
-  st->bin_thr_fixed = a.bin_thr;
-  st->sv_thr_fixed = a.sv_thr;
-  if (!a.keep_modes) {
-    st->count = 0;
-    st->flags = 0;
-  }
+  st->count = 0;
+  st->flags = 0;
   st->found_iter[0] = 0;
   st->found_iter[1] = 1;
   st->iters = 0;
@@ -448,22 +442,17 @@ __device__ __forceinline__ void NextIteration(const Ctx &c, const DevFixed &fx, 
   ip->done = lc->done;
   ip->it = lc->it;
   if (done) return;
-  int32_t B = fx.B_fixed;
-  if (fx.mode == kModeSolve) {
+  int32_t B;
+  if (replay) {
+    B = LoadUniform(&c.log[lc->it]);  // the recorded solve's bins
+  } else {
     const int64_t want = (int64_t(fx.k) - int64_t(count)) * 2 + 1;
     B = int32_t(want > fx.min_bins ? want : fx.min_bins);
-  } else if (replay) {
-    B = LoadUniform(&c.log[lc->it]);  // the recorded solve's bins
   }
   const BParams bp = LoadUniform(&c.btab[B]);
-  FillParams(ip, bp, fx.bits_override > 0 ? fx.bits_override : bp.bits);
-  if (fx.mode == kModeSolve) {
-    ip->bin_thr = bp.bin_thr;
-    ip->sv_thr = bp.sv_thr;
-  } else {
-    ip->bin_thr = fx.bin_thr_fixed;
-    ip->sv_thr = fx.sv_thr_fixed;
-  }
+  FillParams(ip, bp, bp.bits);
+  ip->bin_thr = bp.bin_thr;
+  ip->sv_thr = bp.sv_thr;
   ip->tf = LoadUniform(&c.tfs[lc->it]);
   // ip->q is filled by PublishIteration only: workgroups load the q of
   // their own trial, keeping the struct out of private memory.
