@@ -1446,8 +1446,8 @@ __device__ __forceinline__ void BinFftLarge(const Ctx &c, const IterParams &ip, 
 // bin FFT at B = 101, where this takes 1500.  The per-bin BinInFreq sums do
 // not need the DFT's LDS here, so they are built beside it, between the same
 // two barriers.  Bound by the twiddle reads (one 16-byte LDS gather per pair
-// of pairs): at B = 511 they would take as long as the passes, hence the
-// limit at half of that.
+// of pairs), which grow as B^2.  The limit is the workgroup's size: a thread
+// loads and stages one twiddle; more was not measured.
 // us: a late iteration's launch at n = 2^22, S = 1000 (B = 101, 33 rows)
 // 10.4 -> 7.3; a BinInTime call at n = 2^16, B = 101 12.7 -> 11.0.  Its error
 // is the smaller: 7.3e-16 of the norm against 8.1e-16 (that call, with the
@@ -1462,6 +1462,7 @@ struct DirectLds {
   unsigned long long limbs[4 * kDirectBins];
 };
 static_assert(sizeof(DirectLds) <= kDirectLds, "LDS of the direct bin DFT");
+static_assert(kDirectBins <= kFftThreads, "DirectLoad and DirectStage: one twiddle per thread");
 
 // This thread's x_m, x_(B-m) (conjugated with CONJ_IN) and w_m; issued ahead
 // of whatever else precedes the DFT.  With it, exponents compared in
