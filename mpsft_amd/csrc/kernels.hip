@@ -1272,7 +1272,9 @@ __device__ __forceinline__ double2 FoldAt(const double2 *f, int k, int32_t parts
 }
 
 // CONJ_IN: transform conj(fold) (the adjoint pass feeds conjugated bins,
-// never split); otherwise fold is partial fold 0 of ip.slices.
+// never split); otherwise fold is partial fold 0 of ip.slices.  M is 1024
+// (kDirectBins leaves no smaller one), but stays a variable: as a constant the
+// passes unroll and spill (48 bytes of scratch in k_bin_fft_batch).
 template <bool CONJ_IN>
 __device__ __forceinline__ void BinFftSmall(const Ctx &c, const IterParams &ip, const double2 *fold,
                                             double2 rp, double2 *a) {
