@@ -164,7 +164,10 @@ struct DevState : DevFixed {
   int32_t iters;          // iterations run when the loop stopped
   int32_t stop_stale;     // stale count when the loop stopped
   LoopCounters L[2];
-  IterParams P[2];
+  // on a cache line of its own: every launch starts by loading one of them
+  // (at offset 112 one bin map of B = 101 takes 10.7 us, here 10.4; a solve of
+  // n = 2^22, S = 1000 572 and 561)
+  alignas(128) IterParams P[2];
   int32_t cnt_base[2];  // per parity: |found| when that iteration started
   int32_t pad_[2];
 };
