@@ -383,9 +383,14 @@ Engine::~Engine() {
 // residue's sum is added alike at every R.  Sorted order: batched signals
 // that do not fit the L2s (from 16 MB; 8 MB signals lose nothing to unsorted
 // tiles in XCD order, TileFold) and B of at least 256, below which a line of
-// x hardly serves two samples.  Its tiles are 8 residues wide where the
-// batch still has 384 of them (64 signals, B = 777: R = 4 467 us, R = 8 418)
-// and three fit a CU's LDS.
+// x hardly serves two samples.  It gains with the signals that share the
+// launches and costs little where few do: gather-fold of one solve of 2, 4,
+// 8, 16, 32 signals of n = 2^22, S = 1000 (complex64) unsorted 284, 443, 712,
+// 1277, 2395 us, sorted 289, 443, 691, 1226, 2322; of 8 with S = 300 411 and
+// 429.  Its tiles are 8 residues wide where the batch still has 384 of them
+// (2 signals: 308 us with 8 everywhere, 289 by this rule; 16 signals: R = 2
+// 1289, 4 1251, 8 1228) and three fit a CU's LDS (8 complex128 signals of
+// n = 2^21, S = 500: 630 us with 8 everywhere, 462).
 void Engine::SetTile(BParams *bp, int32_t nlam) const {
   const int32_t forced = forced_R_[bp->B >= kSmallTileB ? 0 : 1];
   const size_t elem = precision_ == MPSFT_MIXED ? sizeof(float2) : sizeof(double2);

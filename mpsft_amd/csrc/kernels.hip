@@ -586,8 +586,9 @@ struct Lags {
 //   phase A gathers the nlam x R distinct samples into LDS (each once),
 //   phase T computes the f x R taps into LDS (each once per iteration),
 //   phase B forms every (row, rho) sum, split over `parts` threads.
-// Bound by phase A: 64 signals of n = 2^22, B = 2001 take 1144 us, 275 us
-// without the gather, and 1190 us with nothing else.  A sample is a 128-byte
+// Bound by phase A: in a probe of the unsorted round-robin form 64 signals of
+// n = 2^22, B = 2001 took 1144 us, 275 without the gather, and no less
+// without the taps or without the sums (1193, 1156).  A sample is a 128-byte
 // line request, at most 62 G/s where lines miss the L2 and 227 G/s where
 // they hit, so what helps is meeting a line again while the L2 holds it:
 //  - XCD order (k_bin_time_batch): each XCD takes a contiguous range of a batch's
@@ -597,11 +598,14 @@ struct Lags {
 //    XCD sweeping x alike.  Position is a B lambda mod n plus a constant of
 //    the residue, so one bucket sort of the lags serves every residue, each
 //    starting at its own bucket; R = 8 keeps 24 residues per CU resident.
-//    64 signals of n = 2^22, complex64, us per launch before / XCD order /
-//    both: B = 2001 1144 / 1056 / 952, 777 537 / 479 / 418, 311 268 / 247 /
-//    240, 101 127 / 114 / 123.  32 of n = 2^20 (8 MB each), B = 201: 73 /
-//    50 / 51.  A signal alone gains nothing from either (its x is read by
-//    all XCDs): 24.3 / 24.9 / 24.2 us at B = 2001.
+// 64 signals of n = 2^22, S = 1000, complex64, us per launch of a solve (by
+// the first signal's B):
+//   B =        2001  1257   809   531   315   195   101
+//   neither    1125   742   552   392   285   220   138
+//   XCD order  1086   677   495   371   275   216   136
+//   both       1006   642   472   368   283   217   136
+// A signal alone gains nothing from either (its x is read by all XCDs): in a
+// batch of one, n = 2^22 ... 2^26, every order is within 2%.
 // Whatever the tile's width, a residue's sum is split and added as the
 // group of G residues it belongs to says, so results do not depend on R.
 // With ip.slices = kSlices the tile is split over the 8 XCDs: its unit s
