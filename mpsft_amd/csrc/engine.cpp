@@ -533,7 +533,12 @@ int Engine::SetTileResidues(int32_t R_wide, int32_t R_narrow) {
     if (!built_[B]) continue;
     BParams &bp = hbtab_[B];
     const int32_t bits = tab_bits_override_ > 0 ? tab_bits_override_ : bp.bits;
-    SetTile(&bp, NumLags(bits, bp.f));
+    const int32_t nlam = NumLags(bits, bp.f);
+    SetTile(&bp, nlam);
+    // for a replay, which may come before the next Reserve
+    tiles_cap_ = std::max(tiles_cap_, (bp.B + bp.R - 1) / bp.R * bp.slices);
+    lds_bin_time_ = std::max(lds_bin_time_, TileLds(bp, nlam, sizeof(double2)));
+    lds_bin_time32_ = std::max(lds_bin_time32_, TileLds(bp, nlam, sizeof(float2)));
   }
   if (d_btab_)
     HIP_OK(hipMemcpy(d_btab_, hbtab_.data(), hbtab_.size() * sizeof(BParams),

@@ -207,6 +207,22 @@ def adjoint(n, k, sigma, seed, trials=1):
                 dot_rel=float(abs(lhs - rhs) / abs(lhs)), dot=abs(lhs))
 
 
+def replay_tiles(n, k, sigma, seed):
+    """A recorded solve replayed with other tile widths, no solve between."""
+    x = signal(n, k, sigma, seed)
+    s = gpu.Solver(n, gpu.solve_options(k, sigma))
+    s.set_record(True)
+    xd = s.upload(x)
+    s.solve(xd, seed)
+    want = s.modes_dict()
+    same = []
+    for residues in (8, 1):
+        s.set_tile_residues(residues)
+        s.replay(xd)
+        same.append(s.modes_dict() == want)
+    return dict(same=same, n_found=len(want))
+
+
 def batch_adjoint(ns, ks, sigma, seeds, precision=0):
     """Batched record + adjoint: per signal the dot-product identity with the
     replayed map, and agreement with the single-signal adjoint."""
@@ -319,5 +335,6 @@ if __name__ == "__main__":
     fn = {"solve": solve, "iterate": iterate, "plan": plan, "batch": batch,
           "adjoint": adjoint, "batch_adjoint": batch_adjoint, "gen": gen, "analyze": analyze,
           "identify": identify, "plan_freq": plan_freq,
-          "plan_freq_first": plan_freq_first, "stream_ends": stream_ends}[case.pop("kind")]
+          "plan_freq_first": plan_freq_first, "stream_ends": stream_ends,
+          "replay_tiles": replay_tiles}[case.pop("kind")]
     print("RESULT " + json.dumps(fn(**case)), flush=True)

@@ -73,6 +73,7 @@ CASES = {
     "adjoint_10007_10_1": dict(kind="adjoint", n=10007, k=10, sigma=1e-6, seed=7, trials=1),
     "batch_adjoint": dict(kind="batch_adjoint", ns=[4096, 8192, 16384], ks=[5, 12, 20],
                           sigma=1e-6, seeds=[3, 4, 5]),
+    "replay_tiles": dict(kind="replay_tiles", n=1 << 14, k=20, sigma=1e-6, seed=7),
     "gen_4099": dict(kind="gen", n=4099, k=7, sigma=0.5, seed=77),
     "gen_65536": dict(kind="gen", n=1 << 16, k=30, sigma=1e-6, seed=123534),
     "analyze": dict(kind="analyze", n=1 << 14, k=40, sigma=1e-5, seed=9),
@@ -189,6 +190,13 @@ def test_emu_replay_and_adjoint(emu_runs, n, k, trials):
     r = result(emu_runs, f"adjoint_{n}_{k}_{trials}")
     assert r["n_found"] >= k and r["same_keys"] and r["replay_err"] == 0.0
     assert r["linear_err"] < 1e-13 and r["dot_rel"] < 1e-12
+
+
+def test_emu_replay_with_another_tile_width(emu_runs):
+    """A tile width set between a recorded solve and its replay: the replay's
+    launch has the LDS and the tiles of the new width."""
+    r = result(emu_runs, "replay_tiles")
+    assert r["n_found"] == 20 and r["same"] == [True, True], r
 
 
 def test_emu_batched_adjoint(emu_runs):

@@ -144,6 +144,24 @@ def test_batch_sorted_tiles_match_single(gpu, n, ks, precision, trials):
             assert abs(got[key] - v) <= TOL * max(abs(v), 1e-2 * top)
 
 
+def test_batch_sorted_tiles_of_every_width(gpu):
+    """Autotuning solves sorted signals with tiles of 1, 2, 4 and 8 residues; the
+    width it leaves gives the modes that the default gave."""
+    from mpsft_amd.signals import make_signal
+    n, ks = 1 << 20, (150, 130)
+    xs = [make_signal(n, k, 1e-6, seed=80 + k)[0] for k in ks]
+    batch = gpu.Batch([n] * 2, [gpu.solve_options(k, 1e-6) for k in ks])
+    xd = batch.upload(xs)
+    iters, status = batch.solve(xd, [3, 4])
+    want = [batch.modes_dict(i) for i in range(2)]
+    assert status == [0, 0] and batch.autotune(xd, [3, 4]) in (0, 1, 2, 4, 8)
+    assert batch.solve(xd, [3, 4]) == (iters, status)
+    for i, m in enumerate(want):
+        got = batch.modes_dict(i)
+        assert set(got) == set(m)
+        assert max(abs(got[q] - v) for q, v in m.items()) <= TOL
+
+
 @pytest.mark.parametrize("bins", [1, 3, 125, 127, 129, 131, 253, 255, 257, 511, 513])
 def test_bin_in_time_dft_paths(gpu, orc, bins):
     """The bin DFT's forms and their edges: direct with one (B <= 127) or two
@@ -206,6 +224,23 @@ def test_mode_counts_follow_every_call(gpu):
         b.solve(xd, seeds)
         sizes = [len(b.modes_dict(i)) for i in range(2)]
     assert sizes == [len(maps[0]), len(maps[1])]
+
+
+def test_replay_with_another_tile_width(gpu):
+    """A tile width set between a recorded solve and its replay."""
+    from mpsft_amd.signals import make_signal
+    n, k = 1 << 16, 60
+    s = gpu.Solver(n, gpu.solve_options(k, 1e-6))
+    s.set_record(True)
+    xd = s.upload(make_signal(n, k, 1e-6, seed=3)[0])
+    s.solve(xd, 4)
+    want = s.modes_dict()
+    for residues in (8, 1, 2):
+        s.set_tile_residues(residues)
+        s.replay(xd)
+        got = s.modes_dict()
+        assert set(got) == set(want)
+        assert max(abs(got[q] - v) for q, v in want.items()) <= TOL
 
 
 def test_modes_after_the_stream_ends(gpu):
