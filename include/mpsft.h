@@ -210,7 +210,8 @@ int mpsft_solver_destroy(mpsft_solver *s);
  * drawn on the host from a std::mt19937 seeded with seed, in the order of
  * Transform(n) (src/integer.cc:44-49) then RandomInt32() % n per trial
  * (src/iterate.cc:103); for n = 2^k the multiplier is drawn odd.
- * Returns the iteration count in *iters. */
+ * Returns the iteration count in *iters.  The stream may be destroyed once
+ * the call has returned. */
 int mpsft_solve(mpsft_solver *s, const void *x_dev, uint32_t seed,
                 int32_t *iters, void *stream);
 
