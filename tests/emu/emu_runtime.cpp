@@ -144,7 +144,12 @@ void Run(const Node &nd) {
   S.nd = &nd;
   S.fibers.resize(nt);
   sched = &S;
-  for (unsigned b = 0; b < nd.grid.x; ++b) {
+  // EMU_ORDER=reverse: the last workgroup and, between barriers, the last
+  // thread first, so that a result which rests on the usual order changes.
+  const char *order = std::getenv("EMU_ORDER");
+  const bool reverse = order && std::strcmp(order, "reverse") == 0;
+  for (unsigned bi = 0; bi < nd.grid.x; ++bi) {
+    const unsigned b = reverse ? nd.grid.x - 1 - bi : bi;
     Block blk;
     if (nd.lds) {
       blk.lds = std::malloc(nd.lds);
@@ -168,7 +173,8 @@ void Run(const Node &nd) {
     }
     for (unsigned live = nt; live > 0;) {
       live = 0;
-      for (unsigned t = 0; t < nt; ++t) {
+      for (unsigned ti = 0; ti < nt; ++ti) {
+        const unsigned t = reverse ? nt - 1 - ti : ti;
         Fiber &f = S.fibers[t];
         if (f.done) continue;
         S.cur = t;

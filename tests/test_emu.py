@@ -60,6 +60,11 @@ CASES = {
     "solve_2": dict(kind="solve", n=1 << 16, k=300, sigma=1e-6, seed=5, precision=0, repeat=1),
     "batch": dict(kind="batch", ns=[4096, 8192, 16384, 4096], ks=[5, 12, 20, 8], sigma=1e-6,
                   seeds=[3, 4, 5, 6]),
+    # the last workgroup and the last thread first
+    "solve_reverse": dict(kind="solve", n=1 << 14, k=60, sigma=3e-6, seed=7, precision=1, repeat=1,
+                          setenv={"EMU_ORDER": "reverse"}),
+    "batch_reverse": dict(kind="batch", ns=[4096, 8192, 16384, 4096], ks=[5, 12, 20, 8], sigma=1e-6,
+                          seeds=[3, 4, 5, 6], setenv={"EMU_ORDER": "reverse"}),
     # the gather-fold split over the 8 XCD slices of x, forced at small n
     "solve_sliced": dict(kind="solve", n=1 << 14, k=40, sigma=3e-6, seed=7, precision=1,
                          repeat=1, setenv={"MPSFT_SLICES": "8"}),
@@ -156,6 +161,16 @@ def test_emu_modes_after_the_stream_ends(emu_runs):
     and the next calls are as after a solve on the null stream."""
     r = result(emu_runs, "stream_ends")
     assert r["n_found"] == 20 and r["same"] == [True] * 4, r
+
+
+def test_emu_in_reverse_order(emu_runs):
+    """Workgroups, and threads between barriers, run last to first: a missing
+    barrier or a workgroup that waits on another's result would show."""
+    r = result(emu_runs, "solve_reverse")
+    assert r["bins"] == r["ref_bins"] and r["same_support"] and r["max_rel_err"] < 1e-10
+    r = result(emu_runs, "batch_reverse")
+    assert r["status"] == [0, 0, 0, 0]
+    assert all(r["same_as_single"]) and all(r["same_as_oracle"]) and r["modes_all_match"]
 
 
 def test_emu_sliced_gather_fold(emu_runs):
